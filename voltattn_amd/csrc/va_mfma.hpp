@@ -73,6 +73,24 @@ __device__ __forceinline__ u32x2 ld64(__amdgpu_buffer_rsrc_t r, uint32_t voff, u
     return __builtin_amdgcn_raw_buffer_load_b64(r, voff, sgpr(soff), VA_LOAD_AUX);
 }
 
+// Max / sum over aligned runs of G = 32 or 64 lanes, in every lane of the run.
+template <int G>
+__device__ __forceinline__ float lanes_max(float x) {
+    x = group_max<16>(x);
+    if constexpr (G == 64) return rows_max(x);
+    unsigned a = __builtin_bit_cast(unsigned, x), b = a;
+    permlane16_swap(a, b);
+    return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+template <int G>
+__device__ __forceinline__ float lanes_sum(float x) {
+    x = group_sum<16>(x);
+    if constexpr (G == 64) return rows_sum(x);
+    unsigned a = __builtin_bit_cast(unsigned, x), b = a;
+    permlane16_swap(a, b);
+    return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+
 // 8 bytes of q4 codes (two dwords, byte order) -> the 8 low nibbles as exact fp16
 // v = n - 8, and the 8 high nibbles as exact fp16 16v (masked in place under the
 // 1024.0 magic: 1024 + 16n - 1152).
@@ -166,6 +184,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
     __shared__ float s_acc[QG][D];
     __shared__ float s_mf[QG], s_lf[QG];
     __shared__ int   s_page[PAGED ? MAX_SPLIT_PAGES : 1];
+    __shared__ __align__(16) int8_t s_qd[3][QG][D];          // q's digits in operand order
+    __shared__ i32x4 s_qc[QG][NG];                          // per column: 2^-sh factor, accumulator starts
     __shared__ int   s_prog[WAVES];                         // tile pair each wave is on (issue priority)
 
     // ---- work-group -> (sequence b, KV head hk, query sub-group, split s)
@@ -217,8 +237,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
             p0 = j0 >> a.page_shift;
             const int np = ((j0 + n - 1) >> a.page_shift) - p0 + 1;
             const int32_t* tab = a.block_table + (size_t)b * a.max_pages + p0;
-            for (int i = (int)threadIdx.x; i < np; i += WAVES * 64) s_page[i] = tab[i];
-            __syncthreads();
+            for (int i = (int)threadIdx.x; i < np; i += WAVES * 64) s_page[i] = tab[i];   // read after the digits' barrier
         }
 
         const uint32_t koff = (uint32_t)(col * ROWB + g * DQ);     // K: row n, quarter g
@@ -282,22 +301,26 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
             __builtin_amdgcn_sched_barrier(0);
         };
 
-        // This lane's q words are loaded ahead of tile 0: vector loads complete
-        // in order, so the digit arithmetic below then overlaps the tile's
-        // latency instead of waiting for it. (Words are taken out of each vector
-        // right after its load.)
-        constexpr int EPQ = D / 4;                // dimensions of a lane quarter
-        uint32_t qwd[EPQ / 2];
-        {
-            const _Float16* qrow = reinterpret_cast<const _Float16*>(a.q) + (size_t)(rt.oh0 + (cq < rt.nq ? cq : 0)) * D;
+        // q as three int8 digits, made once by the work-group: thread t takes
+        // element (query slot, dimension) t, t + NT, .. Its load is issued ahead of
+        // tile 0 (vector loads complete in order, so the digit arithmetic overlaps
+        // the tile's latency). Elements of slots past nq read slot 0 and are unused.
+        // Every wave making all digits for itself took ~750 VALU instructions of
+        // prologue per wave; shared through LDS it is ~100. Same-box A/B on MI355X,
+        // Hq 32 / Hkv 8, D 128, G 32: L 512 q8+ 9.6 -> 8.6 us, q4+ 10.1 -> 8.3, q3+
+        // 10.7 -> 8.6; L 16384 q4+ 13.7 -> 12.1, q3+ 14.8 -> 12.9; L 65536 q3+ 25.7 ->
+        // 24.6, q8+ and q4+ within 0.3.
+        constexpr int NT = WAVES * 64;
+        constexpr int QE = (QG * D + NT - 1) / NT;  // elements per thread
+        uint32_t qh[QE];
 #pragma unroll
-            for (int i = 0; i < EPQ / 8; ++i) {
-                const u32x4 w = *reinterpret_cast<const u32x4*>(qrow + g * EPQ + 8 * i);
-                qwd[4 * i] = w.x; qwd[4 * i + 1] = w.y; qwd[4 * i + 2] = w.z; qwd[4 * i + 3] = w.w;
-            }
+        for (int i = 0; i < QE; ++i) {
+            const int x = (int)threadIdx.x + i * NT;
+            const int qs = x / D;
+            qh[i] = a.q[(size_t)(rt.oh0 + (qs < rt.nq ? qs : 0)) * D + x % D];
         }
         __builtin_amdgcn_sched_barrier(0);
-        load_tile(0, ka, va_, ska, sva);
+        if constexpr (!PAGED) load_tile(0, ka, va_, ska, sva);
 
         // q^T operand of the q.K products: column (cg, cq); k slots of quarter g
         // for MFMA j are dimensions g*DQ + 16j + e, zero outside group cg and for
@@ -305,61 +328,57 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
         // round(q * 2^sh), sh per column putting max|q| in [2^21, 2^22) (every
         // fp16 element within 2^-11 of the maximum is exact; below, the error is
         // under 2^-23 of it), so each digit's dot with the int8 codes is exact
-        // in int32.
-        u32x4 qd[3][NJ];
-        float cf;                                 // qscale * 2^-sh of this column
-        int   qoff[3] = {0, 0, 0};                // q4: -8 * (column sum of each digit)
-        {
-            const int e0 = g * EPQ;               // they all lie in scale group e0 / G
-            const bool use = cq < rt.nq && e0 / G == cg;
-            float qe[EPQ];
-            float lmax = 0.f;
+        // in int32. A column's elements lie on G consecutive lanes.
+        constexpr int EPQ = D / 4;                // dimensions of a lane quarter
 #pragma unroll
-            for (int i = 0; i < EPQ / 8; ++i) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const uint32_t wd = qwd[4 * i + (e >> 1)];
-                    const uint32_t h = (e & 1) ? (wd >> 16) : (wd & 0xFFFFu);
-                    qe[8 * i + e] = use ? h2f(h) : 0.f;
-                    lmax = fmaxf(lmax, fabsf(qe[8 * i + e]));
-                }
-            }
-            const float cmax = rows_max(lmax);          // column maximum over the quarters
+        for (int i = 0; i < QE; ++i) {
+            const int x = (int)threadIdx.x + i * NT;
+            const int qs = x / D, d = x % D;
+            const float qe = h2f(qh[i]);
+            const float cmax = lanes_max<G>(fabsf(qe));
             int sh = 0;
             if (cmax > 0.f) sh = 22 - ((int)((__builtin_bit_cast(uint32_t, cmax) >> 23) & 0xFF) - 126);
-            const float up = __builtin_bit_cast(float, (uint32_t)(127 + sh) << 23);
-            cf = a.qscale * __builtin_bit_cast(float, (uint32_t)(127 - sh) << 23);
-            float dsum[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                uint32_t bq[3][4] = {};
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    // k slot e of MFMA j: q8 dimension 16j + e of the quarter; q4 the
-                    // nibble order of the A operand (low nibbles, then high nibbles)
-                    const int de = !Q4 ? 16 * j + e : (D == 128 ? 2 * e + j : (e < 8 ? 2 * e : 2 * (e - 8) + 1));
-                    const int qi = (int)__builtin_rintf(qe[de] * up);        // |qi| < 2^22
-                    const int d0 = (qi << 24) >> 24;
-                    const int r1 = (qi - d0) >> 8;
-                    const int d1 = (r1 << 24) >> 24;
-                    const int d2 = (r1 - d1) >> 8;                           // |d2| <= 64
-                    bq[0][e >> 2] |= (uint32_t)(d0 & 0xFF) << (8 * (e & 3));
-                    bq[1][e >> 2] |= (uint32_t)(d1 & 0xFF) << (8 * (e & 3));
-                    bq[2][e >> 2] |= (uint32_t)(d2 & 0xFF) << (8 * (e & 3));
-                    dsum[0] += (float)d0;
-                    dsum[1] += (float)d1;
-                    dsum[2] += (float)d2;
-                }
-#pragma unroll
-                for (int k = 0; k < 3; ++k) qd[k][j] = u32x4{bq[k][0], bq[k][1], bq[k][2], bq[k][3]};
+            const int qi = (int)__builtin_rintf(qe * __builtin_bit_cast(float, (uint32_t)(127 + sh) << 23));  // |qi| < 2^22
+            const int d0 = (qi << 24) >> 24;
+            const int r1 = (qi - d0) >> 8;
+            const int d1 = (r1 << 24) >> 24;
+            const int d2 = (r1 - d1) >> 8;                           // |d2| <= 64
+            // byte of dimension d in the operand order: k slot e of MFMA j; q4 takes
+            // the nibble order of the A operand (low nibbles, then high nibbles)
+            const int r = d % EPQ;
+            const int at = d - r + (!Q4 ? r : D == 128 ? 16 * (r & 1) + (r >> 1) : 8 * (r & 1) + (r >> 1));
+            float off[3] = {0.f, 0.f, 0.f};       // codes enter as n = v + 8 (q4), v + 4 (q3)
+            if constexpr (Q4 || Q3) {
+                off[0] = lanes_sum<G>((float)d0) * (Q4 ? -8.f : -4.f);
+                off[1] = lanes_sum<G>((float)d1) * (Q4 ? -8.f : -4.f);
+                off[2] = lanes_sum<G>((float)d2) * (Q4 ? -8.f : -4.f);
             }
-            if constexpr (Q4 || Q3) {             // codes enter as n = v + 8 (q4), v + 4 (q3)
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const float cs = rows_sum(dsum[k]);
-                    qoff[k] = (Q4 ? -8 : -4) * (int)cs;
+            if (QE * NT == QG * D || x < QG * D) {
+                s_qd[0][qs][at] = (int8_t)d0;
+                s_qd[1][qs][at] = (int8_t)d1;
+                s_qd[2][qs][at] = (int8_t)d2;
+                if (d % G == 0) {                 // qscale * 2^-sh of the column, and its accumulator starts
+                    const float c = a.qscale * __builtin_bit_cast(float, (uint32_t)(127 - sh) << 23);
+                    s_qc[qs][d / G] = i32x4{__builtin_bit_cast(int, c), (int)off[0], (int)off[1], (int)off[2]};
                 }
             }
+        }
+        __syncthreads();
+        if constexpr (PAGED) load_tile(0, ka, va_, ska, sva);
+        u32x4 qd[3][NJ];
+        const bool slot_on = cq < rt.nq;
+        const i32x4 qc = slot_on ? s_qc[slot_on ? cq : 0][cg] : i32x4{0, 0, 0, 0};
+        const float cf = __builtin_bit_cast(float, qc.x);
+        const int qoff[3] = {qc.y, qc.z, qc.w};
+        {
+            const bool use = slot_on && g * EPQ / G == cg;
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+                    const u32x4 w = *reinterpret_cast<const u32x4*>(&s_qd[k][use ? cq : 0][g * EPQ + 16 * j]);
+                    qd[k][j] = use ? w : u32x4{0u, 0u, 0u, 0u};
+                }
         }
         const uint32_t magic = [] { uint32_t m; VA_VGPR_CONST(m, 0x64646464); return m; }();
 
