@@ -148,6 +148,22 @@ hipError_t launch_quantize(int bits, int G, const float* x, size_t rows, int D,
 hipError_t launch_dequantize(int bits, int G, const uint8_t* packed, const uint16_t* scales, size_t rows,
                              int D, float* out, hipStream_t stream);
 
+// Division by a divisor fixed for a launch, of dividends below 2^31: with
+// l = ceil(log2 d), mul = floor(2^(31+l) / d) + 1 fits 32 bits and exceeds
+// 2^(31+l) / d by at most 1, so (x * mul) >> (31 + l) is floor(x / d) for every
+// x < 2^31 (Granlund and Montgomery, PLDI 1994).
+struct FastDiv {
+    uint32_t mul, shift, one;   // one: the divisor is 1
+    static FastDiv of(uint32_t d) {
+        uint32_t l = 0;
+        while ((1ull << l) < d) ++l;
+        return FastDiv{(uint32_t)((1ull << (31 + l)) / d + 1), l ? l - 1 : 0u, d == 1 ? 1u : 0u};
+    }
+    __host__ __device__ uint32_t div(uint32_t x) const {
+        return one ? x : (uint32_t)(((uint64_t)x * mul) >> 32) >> shift;
+    }
+};
+
 // Quantize-and-append of n new fp16 rows per (sequence, KV head) into a page
 // pool [num_pages][hkv][page_rows][row bytes] (+ fp16 scales [...][D/G]).
 struct AppendArgs {
@@ -158,6 +174,8 @@ struct AppendArgs {
     uint16_t*       scales;
     int B, hkv, n, D;
     int page_rows, max_pages, num_pages;
+    FastDiv by_n, by_hkv, by_page;   // set by launch_append, as many:
+    bool many;                       // 2^31 rows or more
 };
 hipError_t launch_append(int bits, int G, const AppendArgs& a, hipStream_t stream);
 
