@@ -289,9 +289,11 @@ typedef struct {
 
 /* One decode step of every sequence of the batch: per (sequence, query head)
  * softmax(q.K^T / sqrt(D)) V over that sequence's seq_lens[b] positions.
- * Splits are S ranges of ceil(max_seq_len / S) positions (rounded up to the
- * kernel tile); a sequence shorter than max_seq_len leaves its later splits
- * empty. A sequence of length 0 gives a zero output; a length above
+ * Batches whose lengths can differ enough to matter are cut on the device into
+ * equal shares of the positions that are there, as many as the S splits' ws
+ * holds partials for; otherwise splits are S ranges of ceil(max_seq_len / S)
+ * positions (rounded up to the kernel tile), and a sequence shorter than
+ * max_seq_len leaves its later splits empty. A sequence of length 0 gives a zero output; a length above
  * max_seq_len, or a page id outside the pool on one of its positions, gives
  * NaN for that sequence's heads. S = 0 picks the split count
  * (va_pick_splits_paged). Asynchronous on `stream`. */

@@ -5,7 +5,8 @@
 // A sequence of L positions has ceil(L / BT) tiles of BT positions (one if it is
 // empty) for each of its merge groups (KV head, query sub-group). A merge group
 // counts as its tiles plus COST units (what a work-group spends to begin and end
-// one: lengths, page ids, query operand, first tile's latency, combine, output). The
+// one: lengths, page ids, query operand, first tile's latency, combine, output), unless
+// every merge group fills a run, when each run begins about one item anyway. The
 // units of the batch, numbered by (sequence, merge group, position), are cut into
 // n <= nwg runs whose lengths differ by at most one; work-group w takes run w. A run
 // covers the end of one merge group, any number of whole ones and the start of
@@ -24,6 +25,9 @@
 
 namespace va {
 
+// Positions of a tile of the plan for a kernel whose work-group tile is TB: at least 128.
+constexpr int balance_tile(int TB) { return TB >= 128 ? TB : 128; }
+constexpr int BIG = 1 << 30;
 constexpr int MAX_PIECES = 64;   // pieces of one merge group that one merge takes
 
 template <int CTRL, int ROWS>
@@ -54,6 +58,7 @@ template <int BT, int COST, int MIN_RUN>
 struct Balance {
     const DecodeArgs& a;
     int G;                  // merge groups per sequence
+    int cost;               // COST or 0
     int n, q, r;            // runs; run w starts at unit w*q + w*r/n
     float rn, rt;           // 1 / n; runs per unit
     int at, end;            // units of this work-group's run still to do
@@ -66,9 +71,7 @@ struct Balance {
 
     __device__ __forceinline__ int cap() const { return min(a.L, a.max_pages << a.page_shift); }
     // An invalid length is walked as far as it may be read (its output becomes NaN).
-    __device__ __forceinline__ int units(int x) const {
-        return COST + max(1, (max(0, min(x, cap())) + BT - 1) / BT);
-    }
+    __device__ __forceinline__ int tiles(int x) const { return max(1, (max(0, min(x, cap())) + BT - 1) / BT); }
     // w*r < 2^22 and n < 2^11: half a step's margin is above the product's rounding
     __device__ __forceinline__ int start_of(int w) const { return w * q + (int)(((float)(w * r) + 0.5f) * rn); }
     __device__ __forceinline__ int run_of(int unit) const {
@@ -84,16 +87,22 @@ struct Balance {
         G = a.hkv * a.nsub;
         // lengths 64 at a time; the first 64 stay for the search
         const int x0 = a.seq_lens[min(lane, a.B - 1)];
-        int x = x0, t = lane < a.B ? units(x) : 0, p = wave_scan(t);
-        const int p0 = p;
+        int x = x0, t = lane < a.B ? tiles(x) : 0, p = wave_scan(t);
         int sum = __builtin_amdgcn_readlane(p, 63);
         int most = __builtin_amdgcn_readlane(wave_scan_max(t), 63);
+        int least = BIG - __builtin_amdgcn_readlane(wave_scan_max(lane < a.B ? BIG - t : 0), 63);
         for (int c = 64; c < a.B; c += 64) {
-            const int y = c + lane < a.B ? units(a.seq_lens[min(c + lane, a.B - 1)]) : 0;
+            const bool in = c + lane < a.B;
+            const int y = in ? tiles(a.seq_lens[min(c + lane, a.B - 1)]) : 0;
             sum += __builtin_amdgcn_readlane(wave_scan(y), 63);
             most = max(most, __builtin_amdgcn_readlane(wave_scan_max(y), 63));
+            least = min(least, BIG - __builtin_amdgcn_readlane(wave_scan_max(in ? BIG - y : 0), 63));
         }
-        const int T = sum * G;
+        cost = (long long)least * a.nwg >= (long long)sum * G ? 0 : COST;
+        const int T = (sum + cost * a.B) * G;
+        most += cost;
+        t += lane < a.B ? cost : 0;
+        p += min(lane + 1, a.B) * cost;
         n = min(a.nwg, max(1, T / max(MIN_RUN, (most + MAX_PIECES - 3) / (MAX_PIECES - 2))));
         at = end = 0;
         const int w = (int)blockIdx.x;
@@ -105,7 +114,6 @@ struct Balance {
         at = start_of(w);
         end = w == n - 1 ? T : start_of(w + 1);
         base = 0;
-        p = p0;
         for (int c = 0;;) {                                  // ends: at < T, the units' total
             const uint64_t hit = __builtin_amdgcn_ballot_w64((base + p) * G > at);
             if (hit) {
@@ -120,26 +128,33 @@ struct Balance {
             c += 64;
             if (c >= a.B) { at = end; return; }
             x = a.seq_lens[min(c + lane, a.B - 1)];
-            t = c + lane < a.B ? units(x) : 0;
+            t = c + lane < a.B ? tiles(x) + cost : 0;
             p = wave_scan(t);
         }
         ahead = a.seq_lens[min(b + 1, a.B - 1)];
         const int off = at - base * G;
-        g = off / ub;
+        g = (int)((float)off * __builtin_amdgcn_rcpf((float)ub));   // at most a step off
+        while (g > 0 && g * ub > off) --g;
+        while ((g + 1) * ub <= off) ++g;
+        g = uniform(g);
         u0 = off - g * ub;
     }
 
     // The next item of the run, or false.
     __device__ __forceinline__ bool next() {
         const int u1 = min(ub, u0 + end - at);               // past the last unit here
-        if (at >= end || u1 <= COST) return false;           // done, or the run ends before a tile
-        const int gs = base * G + g * ub;                    // the merge group's first unit
-        first = run_of(gs + COST);
-        pieces = run_of(gs + ub - 1) - first + 1;
-        t0 = max(0, u0 - COST);
-        cnt = u1 - COST - t0;
+        if (at >= end || u1 <= cost) return false;           // done, or the run ends before a tile
+        t0 = max(0, u0 - cost);
+        cnt = u1 - cost - t0;
         at += u1 - u0;
         return true;
+    }
+    // Where the merge group of the current item starts, and its pieces: needed at the
+    // item's end only, so the caller asks while the first loads are under way.
+    __device__ __forceinline__ void locate() {
+        const int gs = base * G + g * ub;                    // the merge group's first unit
+        first = run_of(gs + cost);
+        pieces = run_of(gs + ub - 1) - first + 1;
     }
     // Past the current item: it ended its merge group or the run.
     __device__ __forceinline__ void advance() {
@@ -149,7 +164,7 @@ struct Balance {
             base += ub;
             ++b;
             len = ahead;
-            ub = units(len);
+            ub = tiles(len) + cost;
             ahead = a.seq_lens[min(b + 1, a.B - 1)];
         }
     }

@@ -119,6 +119,39 @@ static int max_tile() {
     return std::max(std::max(ex_tile<KIND, D, 1>(), ex_tile<KIND, D, 2>()), ex_tile<KIND, D, 4>());
 }
 
+// Balanced paged forms (va_balance.hpp): work-groups per CU and waves per work-group.
+// Matrix cores: one 8-wave group per CU; two 4-wave groups for q4 and q3 once there are
+// more merge groups than CUs, when a run begins several of them and one group's start
+// and end hide behind the other's loop (batch of 64 up to 3000 positions, Hq 32 / Hkv 8:
+// q4 36.0 -> 30.5 us, q3 39.2 -> 34.2; eight waves stay better for q8, uniform batch of 32
+// x 4096 56.3 -> 50.3, and with fewer merge groups). Vector ALU with one query slot
+// (4-wave groups): two per CU (batch of 64 up to 2000, Hkv 8: q8 25.1 -> 20.3 us, q3 24.9 ->
+// 20.8, f16 32.9 -> 31.1; batch of 16 up to 8192 q8 17.4 -> 15.4), one where fewer merge
+// groups meet longer items (q4 at D 128 16.5 against 18.0, D 64 q8 13.5 against 15.1).
+// Grouped f16 and q3 at D = 64 (8-wave groups): one (f16 26.1 against 34.1).
+static int bal_waves(int kind, long long groups) { return kind != KQ8 && groups >= 256 ? 4 : 8; }
+
+template <int KIND, int D>
+static int bal_tile(int qg) {
+    return balance_tile(qg == 1 ? ex_tile<KIND, D, 1>() : qg == 2 ? ex_tile<KIND, D, 2>() : ex_tile<KIND, D, 4>());
+}
+
+int balanced_groups(int kind, int D, int qg, long long groups, int cus) {
+    if (mfma_form(kind, D, qg)) return cus * 8 / bal_waves(kind, groups);
+    const bool two = qg == 1 && (groups >= cus || (D == 128 && kind != KQ4));
+    return two ? 2 * cus : cus;
+}
+
+int balanced_tile(int kind, int D, int qg, long long groups) {
+    if (mfma_form(kind, D, qg)) return 32 * bal_waves(kind, groups);
+    switch (kind) {
+        case KF16: return D == 128 ? bal_tile<KF16, 128>(qg) : bal_tile<KF16, 64>(qg);
+        case KQ8:  return D == 128 ? bal_tile<KQ8, 128>(qg) : bal_tile<KQ8, 64>(qg);
+        case KQ4:  return D == 128 ? bal_tile<KQ4, 128>(qg) : bal_tile<KQ4, 64>(qg);
+        default:   return D == 128 ? bal_tile<KQ3, 128>(qg) : bal_tile<KQ3, 64>(qg);
+    }
+}
+
 int tile_positions_ex(int kind, int D) {
     switch (kind) {
         case KF16: return D == 128 ? max_tile<KF16, 128>() : max_tile<KF16, 64>();
@@ -161,7 +194,13 @@ template <int KIND, int D, int G, int QG, bool PAGED>
 static hipError_t launch_ex(int groups, const DecodeArgs& a, hipStream_t st) {
     constexpr int PTB = Tile<KIND, D>::PPW * 4 * 4;   // the paged form's work-group tile (a power of two)
     if constexpr (VA_EX_PHASED_PAGED && QG == 1 && PAGED && (KIND == KF16 || (VA_EX_PHASED_PAGED_Q8 && KIND == KQ8))) {
-        if ((1 << a.page_shift) >= PTB && a.chunk % PTB == 0) {
+        const bool fits = (1 << a.page_shift) >= PTB;   // balanced tiles are multiples of PTB
+        if (fits && a.nwg > 0) {
+            hipLaunchKernelGGL((decode_phased<KIND, D, G, 4, 4, 1, true, true>), dim3((unsigned)a.nwg), dim3(256), 0, st,
+                               VA_TILED_ARGS(a));
+            return hipGetLastError();
+        }
+        if (fits && a.chunk % PTB == 0) {
             hipLaunchKernelGGL((decode_phased<KIND, D, G, 4, 4, 1, true>), dim3((unsigned)(groups * a.S)), dim3(256),
                                0, st, VA_TILED_ARGS(a));
             return hipGetLastError();
@@ -172,6 +211,17 @@ static hipError_t launch_ex(int groups, const DecodeArgs& a, hipStream_t st) {
                            dim3(VA_EX_PH_WAVES * 64), 0, st, VA_TILED_ARGS(a));
         return hipGetLastError();
     } else if constexpr (mfma_kind_c<KIND, D> && QG >= 2) {
+        if constexpr (PAGED) {
+            if (a.nwg > 0) {
+                if (bal_waves(KIND, groups) == 4)
+                    hipLaunchKernelGGL((decode_mfma<KIND, D, G, 4, QG, true, true>), dim3((unsigned)a.nwg), dim3(256), 0,
+                                       st, a);
+                else
+                    hipLaunchKernelGGL((decode_mfma<KIND, D, G, 8, QG, true, true>), dim3((unsigned)a.nwg), dim3(512), 0,
+                                       st, a);
+                return hipGetLastError();
+            }
+        }
         hipLaunchKernelGGL((decode_mfma<KIND, D, G, MFMA_WAVES, QG, PAGED>),
                            dim3((unsigned)(groups * a.S)), dim3(MFMA_WAVES * 64), 0, st, a);
         return hipGetLastError();
@@ -181,6 +231,13 @@ static hipError_t launch_ex(int groups, const DecodeArgs& a, hipStream_t st) {
         using Cfg = ExCfg<KIND, QG>;
         constexpr int U = ex_unroll<KIND, D, QG>();
         static_assert(Tile<KIND, D>::PPW * U <= 64, "a wave tile must fit the smallest page");
+        if constexpr (PAGED) {
+            if (a.nwg > 0) {
+                hipLaunchKernelGGL((decode_tiled<KIND, D, G, U, Cfg::WAVES, QG, true, Cfg::MINB, true>),
+                                   dim3((unsigned)a.nwg), dim3(Cfg::WAVES * 64), 0, st, VA_TILED_ARGS(a));
+                return hipGetLastError();
+            }
+        }
         hipLaunchKernelGGL((decode_tiled<KIND, D, G, U, Cfg::WAVES, QG, PAGED, Cfg::MINB>),
                            dim3((unsigned)(groups * a.S)), dim3(Cfg::WAVES * 64), 0, st, VA_TILED_ARGS(a));
         return hipGetLastError();

@@ -97,6 +97,15 @@ struct Route {
     int oh0;   // global index of query slot 0: rows of q, out and ws
 };
 
+// Plain fp32 partials of one merge group in the counted protocol: partial (q, s)
+// is o[0..D), m, l at base + q*qs + s*ss (floats); S splits take part, this
+// work-group's is s.
+struct PartStore {
+    float* base;
+    int ss, qs;
+    int S, s;
+};
+
 // Work-group of NT threads; thread t < D holds acc[q] = o[t] of query slot q's
 // partial, and M[q], ls[q] (slots >= nq are ignored).
 //
@@ -287,14 +296,12 @@ __device__ void finish_tagged(const DecodeArgs& a, const Route& rt, const float 
 // flagged with l = NaN) gives NaN, and so does a count that never completes
 // within the poll bound. Needs S <= 64.
 template <int D, int NT, int QG>
-__device__ void finish_counted(const DecodeArgs& a, const Route& rt, const float (&M)[QG],
+__device__ void finish_counted(const DecodeArgs& a, const Route& rt, const PartStore& ps, const float (&M)[QG],
                                const float (&ls)[QG], const float (&acc)[QG]) {
     constexpr int NW = NT / 64;
-    constexpr int PSF = D + 4;                   // floats per partial: o[D], m, l, 2 spare (16-byte rows)
-    constexpr uint32_t PB = PSF * 4;
-    static_assert(PSF <= PARTF_STRIDE, "partial store");
+    const uint32_t PB = (uint32_t)ps.ss * 4u;    // bytes from one split's partial to the next
     const int t = (int)threadIdx.x;
-    const int S = a.S, s = rt.s;
+    const int S = ps.S, s = ps.s;
     constexpr int WQ = NW / QG;
     static_assert(NW >= QG && NW % QG == 0, "whole waves per query slot");
     __shared__ int   s_last, s_bad;
@@ -302,12 +309,11 @@ __device__ void finish_counted(const DecodeArgs& a, const Route& rt, const float
     __shared__ float s_fold[QG][WQ][D];
     __shared__ float s_lsum[QG];
     unsigned* line = g_tickets + ((size_t)a.ticket_slot * TICKET_MAXH + rt.mg) * TICKET_STRIDE;
-    float* base = g_partf + (size_t)a.ticket_slot * PART_CAP * PARTF_STRIDE + (size_t)rt.mg * QG * S * PSF;
     if (t < D) {
 #pragma unroll
         for (int q = 0; q < QG; ++q) {
             if (q >= rt.nq) break;
-            float* mine = base + ((size_t)q * S + s) * PSF;
+            float* mine = ps.base + (size_t)q * ps.qs + (size_t)s * ps.ss;
             store_dev(mine + t, acc[q]);
             if (t == 0) {
                 store_dev(mine + D, M[q]);
@@ -360,7 +366,7 @@ __device__ void finish_counted(const DecodeArgs& a, const Route& rt, const float
     const int jl  = min(lane, S - 1);
     const bool in_s = lane < S, own = lane == s;
     if (qw < rt.nq) {                            // wave-uniform
-        const __amdgpu_buffer_rsrc_t rp = make_rsrc(base + (size_t)qw * S * PSF, (uint32_t)S * PB);
+        const __amdgpu_buffer_rsrc_t rp = make_rsrc(ps.base + (size_t)qw * ps.qs, (uint32_t)(S - 1) * PB + (D + 2) * 4u);
         const int nsw = (S - sw + WQ - 1) / WQ;  // splits folded by this wave
         const int ni  = (nsw + SPL - 1) / SPL;   // load instructions
         // The words are taken out of each 16-byte vector right after its load
@@ -478,7 +484,13 @@ __device__ void finish_partial(const DecodeArgs& a, const Route& rt, const float
         return;
     }
     if constexpr (QG == 1) finish_tagged<D, NT, QG>(a, rt, M, ls, acc, epoch);
-    else finish_counted<D, NT, QG>(a, rt, M, ls, acc);
+    else {
+        constexpr int PSF = D + 4;               // o[D], m, l, 2 spare: 16-byte rows
+        static_assert(PSF <= PARTF_STRIDE, "partial store");
+        const PartStore ps{g_partf + (size_t)a.ticket_slot * PART_CAP * PARTF_STRIDE + (size_t)rt.mg * QG * S * PSF,
+                           PSF, S * PSF, S, s};
+        finish_counted<D, NT, QG>(a, rt, ps, M, ls, acc);
+    }
 }
 
 } // namespace va

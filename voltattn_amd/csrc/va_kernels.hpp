@@ -32,6 +32,10 @@ struct DecodeArgs {
     int   max_pages;        // block-table row length
     int   page_shift;       // log2(page_rows)
     int   num_pages;        // pages in the pool (ids outside [0, num_pages) are rejected)
+    // balanced paged form (va_balance.hpp): work-groups that share the batch's tiles; 0: one
+    // work-group per (merge group, split). Its partials go to ws, its merge needs a ticket slot.
+    int   nwg;
+    int   B;                // sequences in the batch
 };
 
 // Launch of the tiled decode kernel: the leading scalar arguments (preloaded
@@ -91,6 +95,10 @@ hipError_t launch_decode_ex(int kind, int D, int G, int qg, bool paged, int grou
 // work-group tile (positions per iteration) of the grouped/paged kernels.
 int max_query_slots(int kind, int D);
 int tile_positions_ex(int kind, int D);
+// Work-groups of a balanced paged launch (DecodeArgs::nwg) over `groups` merge
+// groups on `cus` CUs, and the positions of its tiles.
+int balanced_groups(int kind, int D, int qg, long long groups, int cus);
+int balanced_tile(int kind, int D, int qg, long long groups);
 // Work-groups per CU the grouped/paged launch of (kind, QG) is built for.
 int ex_groups_per_cu(int kind, int D, int qg);
 

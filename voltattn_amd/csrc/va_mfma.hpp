@@ -48,6 +48,7 @@
 // finish_partial for the partials / fused merge.
 #pragma once
 #include "va_codec.hpp"
+#include "va_balance.hpp"
 #include "va_fused.hpp"
 #include "va_tiled.hpp"
 
@@ -151,8 +152,8 @@ __device__ __forceinline__ void q3_to_bytes(const u32x4& w, uint32_t (&b)[8]) {
     b[7] = q3_spread4(w.z >> 20);
 }
 
-template <int KIND, int D, int G, int WAVES, int QG, bool PAGED>
-__global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
+template <int KIND, int D, int G, int WAVES, int QG, bool PAGED, bool BAL = false>
+__global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void decode_mfma(DecodeArgs a) {
     static_assert(KIND == KQ8 || KIND == KQ4 || (KIND == KQ3 && D == 128),
                   "matrix-core form: q8 and q4 rows, and q3 rows at D = 128");
     constexpr bool Q4  = KIND == KQ4;
@@ -188,33 +189,50 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
     __shared__ i32x4 s_qc[QG][NG];                          // per column: 2^-sh factor, accumulator starts
     __shared__ int   s_prog[WAVES];                         // tile pair each wave is on (issue priority)
 
-    // ---- work-group -> (sequence b, KV head hk, query sub-group, split s)
-    Route rt;
-    rt.mg = (int)blockIdx.x / a.S;
-    rt.s  = (int)blockIdx.x - rt.mg * a.S;
-    const int sub = rt.mg % a.nsub;
-    const int hk  = (rt.mg / a.nsub) % a.hkv;
-    const int b   = (rt.mg / a.nsub) / a.hkv;
-    rt.nq  = min(QG, a.qgroup - sub * QG);
-    rt.oh0 = (b * a.hkv + hk) * a.qgroup + sub * QG;
-    const int s = rt.s;
-    const unsigned epoch = read_epoch<QG>(a, rt.mg);
+    static_assert(!BAL || PAGED, "balanced runs: paged batches");
+    Balance<TB, 256 / TB, 256 / TB> bal(BAL, a);
     const int wave = uniform((int)(threadIdx.x >> 6));
-    const int lane = (int)(threadIdx.x & 63);
+
+    do {
+    if (BAL && !bal.next()) return;
+    int tid = (int)threadIdx.x;
+    if constexpr (BAL) asm volatile("" : "+v"(tid));   // per-lane values are not carried from item to item
+    const int lane = tid & 63;
     const int g    = lane >> 4;                  // quarter
     const int col  = lane & 15;                  // column / row-in-block
     const int cg   = col / QP;                   // scale group of this column
     const int cq   = col % QP;                   // query slot of this column
+    // ---- work-group -> (sequence b, KV head hk, query sub-group, split s), or
+    // the next item of a balanced run
+    Route rt;
+    rt.mg = BAL ? bal.b * bal.G + bal.g : (int)blockIdx.x / a.S;
+    rt.s  = BAL ? 0 : (int)blockIdx.x - rt.mg * a.S;
+    int sub = 0, hk, b;
+    if constexpr (BAL) {
+        b = bal.b;
+        hk = bal.g;
+        if (a.nsub > 1) {
+            hk = bal.g / a.nsub;
+            sub = bal.g - hk * a.nsub;
+        }
+    } else {
+        sub = rt.mg % a.nsub;
+        hk  = (rt.mg / a.nsub) % a.hkv;
+        b   = (rt.mg / a.nsub) / a.hkv;
+    }
+    rt.nq  = min(QG, a.qgroup - sub * QG);
+    rt.oh0 = (b * a.hkv + hk) * a.qgroup + sub * QG;
+    const unsigned epoch = read_epoch<QG>(a, rt.mg);
 
     int L = a.L;
     bool bad = false;
     if constexpr (PAGED) {
-        const int cap = min(a.L, min(a.S * a.chunk, a.max_pages << a.page_shift));
-        L = a.seq_lens[b];
+        const int cap = BAL ? bal.cap() : min(a.L, min(a.S * a.chunk, a.max_pages << a.page_shift));
+        L = BAL ? bal.len : a.seq_lens[b];
         if (L > cap || L < 0) { bad = true; L = L < 0 ? 0 : cap; }   // outside [0, max_seq_len]: NaN output
     }
-    const int j0 = s * a.chunk;
-    const int n  = min(L - j0, a.chunk);
+    const int j0 = BAL ? bal.t0 * TB : rt.s * a.chunk;
+    const int n  = min(L - j0, BAL ? bal.cnt * TB : a.chunk);
 
     // Per lane, for its column (cg, cq): running max mq and weight sum lsum of
     // query slot cq, and the row exponent ex (the P.V operands and the o row of
@@ -224,6 +242,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) o[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    if (BAL && n <= 0) bal.locate();
     if (n > 0) {
         const int niter = (n + TB - 1) / TB;
         const size_t   row0  = PAGED ? 0 : (size_t)hk * a.L + j0;
@@ -237,7 +256,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
             p0 = j0 >> a.page_shift;
             const int np = ((j0 + n - 1) >> a.page_shift) - p0 + 1;
             const int32_t* tab = a.block_table + (size_t)b * a.max_pages + p0;
-            for (int i = (int)threadIdx.x; i < np; i += WAVES * 64) s_page[i] = tab[i];   // read after the digits' barrier
+#pragma unroll 1
+            for (int i = tid; i < np; i += WAVES * 64) s_page[i] = tab[i];   // read after the digits' barrier
         }
 
         const uint32_t koff = (uint32_t)(col * ROWB + g * DQ);     // K: row n, quarter g
@@ -305,17 +325,12 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
         // element (query slot, dimension) t, t + NT, .. Its load is issued ahead of
         // tile 0 (vector loads complete in order, so the digit arithmetic overlaps
         // the tile's latency). Elements of slots past nq read slot 0 and are unused.
-        // Every wave making all digits for itself took ~750 VALU instructions of
-        // prologue per wave; shared through LDS it is ~100. Same-box A/B on MI355X,
-        // Hq 32 / Hkv 8, D 128, G 32: L 512 q8+ 9.6 -> 8.6 us, q4+ 10.1 -> 8.3, q3+
-        // 10.7 -> 8.6; L 16384 q4+ 13.7 -> 12.1, q3+ 14.8 -> 12.9; L 65536 q3+ 25.7 ->
-        // 24.6, q8+ and q4+ within 0.3.
         constexpr int NT = WAVES * 64;
         constexpr int QE = (QG * D + NT - 1) / NT;  // elements per thread
         uint32_t qh[QE];
 #pragma unroll
         for (int i = 0; i < QE; ++i) {
-            const int x = (int)threadIdx.x + i * NT;
+            const int x = tid + i * NT;
             const int qs = x / D;
             qh[i] = a.q[(size_t)(rt.oh0 + (qs < rt.nq ? qs : 0)) * D + x % D];
         }
@@ -332,7 +347,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
         constexpr int EPQ = D / 4;                // dimensions of a lane quarter
 #pragma unroll
         for (int i = 0; i < QE; ++i) {
-            const int x = (int)threadIdx.x + i * NT;
+            const int x = tid + i * NT;
             const int qs = x / D, d = x % D;
             const float qe = h2f(qh[i]);
             const float cmax = lanes_max<G>(fabsf(qe));
@@ -365,6 +380,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
         }
         __syncthreads();
         if constexpr (PAGED) load_tile(0, ka, va_, ska, sva);
+        if constexpr (BAL) bal.locate();
         u32x4 qd[3][NJ];
         const bool slot_on = cq < rt.nq;
         const i32x4 qc = slot_on ? s_qc[slot_on ? cq : 0][cg] : i32x4{0, 0, 0, 0};
@@ -622,10 +638,12 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
     if constexpr (PAGED) any_bad = __syncthreads_or(bad);
     else __syncthreads();
     // fold the WAVES partials of each (query slot, dimension), one per thread
-    const int t = (int)threadIdx.x;
-    static_assert(QG * D <= WAVES * 64, "one thread per (query slot, dimension)");
-    if (t < QG * D) {
-        const int q = t / D, d = t - (t / D) * D;
+    const int t = tid;
+#pragma unroll
+    for (int k = 0; k < (QG * D + WAVES * 64 - 1) / (WAVES * 64); ++k) {
+        const int i = t + k * WAVES * 64;
+        if (QG * D % (WAVES * 64) != 0 && i >= QG * D) break;
+        const int q = i / D, d = i - (i / D) * D;
         float m = s_m[q][0];
 #pragma unroll
         for (int w = 1; w < WAVES; ++w) m = fmaxf(m, s_m[q][w]);
@@ -650,7 +668,13 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_mfma(DecodeArgs a) {
         ls[q] = s_lf[q];
         acc[q] = t < D ? s_acc[q][t] : 0.f;
     }
-    finish_partial<D, WAVES * 64, QG>(a, rt, M, ls, acc, epoch);
+    if constexpr (BAL) {
+        finish_item<D, WAVES * 64, QG>(a, rt, bal, M, ls, acc);
+        bal.advance();
+    } else {
+        finish_partial<D, WAVES * 64, QG>(a, rt, M, ls, acc, epoch);
+    }
+    } while (BAL);
 }
 
 } // namespace va

@@ -45,14 +45,14 @@ namespace va {
 // round at QG > 1 holds 8192/QG positions, so its scores take the same 32 KB.
 constexpr int PHASED_ROUND_ROWS = 8192;
 
-template <int KIND, int D, int G, int U, int WAVES, int QG = 1, bool PAGED = false>
+template <int KIND, int D, int G, int U, int WAVES, int QG = 1, bool PAGED = false, bool BAL = false>
 __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
     const uint8_t* k, const uint8_t* v, const uint16_t* sk, const uint16_t* sv,
     int L_, int S_, int chunk_, int slot_, const uint16_t* q, void* dst, DecodeArgs rest) {
     DecodeArgs a = rest;
     a.k = k; a.v = v; a.sk = sk; a.sv = sv; a.q = q;
     a.out = static_cast<uint16_t*>(dst);
-    a.ws = static_cast<float*>(dst);
+    a.ws = BAL ? rest.ws : static_cast<float*>(dst);   // dst is out in a fused call
     a.L = L_; a.S = S_; a.chunk = chunk_; a.ticket_slot = slot_;
     a.qscale = qscale_of<D>();
     using T = Tile<KIND, D>;
@@ -82,12 +82,27 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
     __shared__ float s_score[WAVES][QG][RT * TW];  // raw scores of the wave's rows in the round
     __shared__ int s_page[PAGED ? MAX_SPLIT_PAGES : 1];
 
-    // work-group -> (KV head hk, query sub-group, split s)
+    static_assert(!BAL || PAGED, "balanced runs: paged batches");
+    constexpr int BT = balance_tile(TB);
+    Balance<BT, 256 / BT, 256 / BT> bal(BAL, a);
+    do {
+    if (BAL && !bal.next()) return;
+    // work-group -> (KV head hk, query sub-group, split s), or the next item of a balanced run
     Route rt;
-    rt.mg  = (int)blockIdx.x / a.S;
-    rt.s   = (int)blockIdx.x - rt.mg * a.S;
+    rt.mg  = BAL ? bal.b * bal.G + bal.g : (int)blockIdx.x / a.S;
+    rt.s   = BAL ? 0 : (int)blockIdx.x - rt.mg * a.S;
     int hk = rt.mg, b = 0;
-    if constexpr (PAGED) {                       // sequence b, KV head hk, one query head
+    if constexpr (BAL) {
+        b = bal.b;
+        hk = bal.g;
+        int sub = 0;
+        if (a.nsub > 1) {
+            hk = bal.g / a.nsub;
+            sub = bal.g - hk * a.nsub;
+        }
+        rt.nq  = 1;
+        rt.oh0 = (b * a.hkv + hk) * a.qgroup + sub;
+    } else if constexpr (PAGED) {                // sequence b, KV head hk, one query head
         const int sub = rt.mg % a.nsub;
         const int r   = rt.mg / a.nsub;
         hk = r % a.hkv;
@@ -103,10 +118,11 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
         rt.nq  = min(QG, a.qgroup - sub * QG);
         rt.oh0 = hk * a.qgroup + sub * QG;
     }
-    const int s = rt.s;
-    const unsigned epoch = read_epoch<QG>(a, rt.mg);
-    const int wave = uniform((int)(threadIdx.x >> 6));
-    const int lane = (int)(threadIdx.x & 63);
+    const unsigned epoch = BAL ? 0u : read_epoch<QG>(a, rt.mg);
+    int tid = (int)threadIdx.x;
+    if constexpr (BAL) asm volatile("" : "+v"(tid));   // per-lane values are not carried from item to item
+    const int wave = uniform(tid >> 6);
+    const int lane = tid & 63;
     const int sl   = lane % LP;                  // lane within its row
     const int pw   = lane / LP;                  // row slot within a wave load
     const int grp  = (sl * EPL) / G;             // scale group of this lane
@@ -114,12 +130,12 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
     int L = a.L;
     bool bad = false;                            // invalid input: the output becomes NaN
     if constexpr (PAGED) {
-        const int cap = min(a.L, min(a.S * a.chunk, a.max_pages << a.page_shift));
-        L = a.seq_lens[b];
+        const int cap = BAL ? bal.cap() : min(a.L, min(a.S * a.chunk, a.max_pages << a.page_shift));
+        L = BAL ? bal.len : a.seq_lens[b];
         if (L > cap || L < 0) { bad = true; L = L < 0 ? 0 : cap; }   // outside [0, max_seq_len]: NaN output
     }
-    const int j0 = s * a.chunk;
-    const int n  = min(L - j0, a.chunk);         // rows of this split (<= 0: empty)
+    const int j0 = BAL ? bal.t0 * BT : rt.s * a.chunk;
+    const int n  = min(L - j0, BAL ? bal.cnt * BT : a.chunk);   // rows of this split (<= 0: empty)
 
     float m[QG], l[QG];
     float o[QG][EPL];
@@ -152,7 +168,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
             p0 = j0 >> a.page_shift;
             const int np = ((j0 + n - 1) >> a.page_shift) - p0 + 1;
             const int32_t* tab = a.block_table + (size_t)b * a.max_pages + p0;
-            for (int i = (int)threadIdx.x; i < np; i += WAVES * 64) s_page[i] = tab[i];
+#pragma unroll 1
+            for (int i = tid; i < np; i += WAVES * 64) s_page[i] = tab[i];
             __syncthreads();
             pnext = s_page[0];                   // stage 0: the split's first tile
         }
@@ -222,6 +239,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
         };
 
         load_stage(0, xa, sa);
+        if constexpr (BAL) bal.locate();
 
         // q slices of this lane (dims [sl*EPL, sl*EPL + EPL)); query slots past
         // nq read query slot 0 (their results are dropped)
@@ -370,7 +388,16 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
         for (int q = 0; q < QG; ++q) fix_finish<C>(o[q], vsum[q], std::make_integer_sequence<int, EPL>{});
     }
 
-    group_finish<D, LP, EPL, WAVES, QG, PAGED>(a, rt, m, l, o, bad, epoch);
+    if (BAL && n <= 0) bal.locate();
+    group_finish<D, LP, EPL, WAVES, QG, PAGED>(m, l, o, bad, [&](auto& M, auto& ls, auto& acc) {
+        if constexpr (BAL) finish_item<D, WAVES * 64, QG>(a, rt, bal, M, ls, acc);
+        else finish_partial<D, WAVES * 64, QG>(a, rt, M, ls, acc, epoch);
+    });
+    if constexpr (BAL) {
+        bal.advance();
+        __syncthreads();                         // the fold has read LDS that the next item writes
+    }
+    } while (BAL);
 }
 
 } // namespace va

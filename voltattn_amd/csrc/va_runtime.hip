@@ -481,14 +481,48 @@ void splits_ex(int kind, int D, int qg, int groups, int max_len, int S_req, int*
     *S = S_req > 0 ? S_req : std::max(1, (max_len + *chunk - 1) / *chunk);
 }
 
+// Work-groups of the balanced form (va_balance.hpp) for a paged batch, or 0 where
+// every merge group is cut into S splits of the longest sequence instead.
+//
+// The plan costs a launch 1 to 2 us, so it is for batches whose uneven lengths can cost
+// more than that: more merge groups than CUs (a split each leaves a half-empty last
+// round), or at least 2048 positions per CU. Measured on MI355X against the splits, D
+// 128, lengths spread over 1/32 .. 1 of the longest: q8 batch of 48 up to 16384, Hq 32 /
+// Hkv 8 171 -> 104 us; q4 64 up to 3000 43.7 -> 30.6; f16 16 up to 8000 63.8 -> 26.1; Hq =
+// Hkv = 8, 16 up to 8192 f16 56.6 -> 22.6, q8 39.6 -> 15.4; Hq 64 / Hkv 8 q4 63.1 -> 26.7.
+// Equal lengths: 40 x 2048 q8 53.8 -> 41, 32 x 4096 52.0 -> 51.2, 8 x 16384 51.8 -> 53.2;
+// below the line 4 x 8192 with Hq = Hkv = 8 would be 15.0 -> 17.2, 2 x 512 6.7 -> 9.0.
+//
+// Also 0: one sequence (its length is what the splits are made for), more merge groups
+// than ticket lines, a run that could span more pages than a work-group stages, or a
+// workspace of S splits (S = 0: any) too small for the pieces of one run per CU.
+int balanced_wgs(int kind, const va_paged_shape* sh, int qg, long long groups, int S) {
+    int cus = cu_count();
+    if (cus <= 0) cus = 256;
+    if (sh->B < 2 || groups > va::TICKET_MAXH) return 0;
+    if (groups <= cus && groups * sh->max_seq_len < 2048LL * cus) return 0;
+    long long n = va::balanced_groups(kind, sh->D, qg, groups, cus);
+    if (S > 0) n = std::min(n, (long long)sh->B * sh->Hq * S / qg - groups);
+    if (n < cus) return 0;
+    const long long bt = va::balanced_tile(kind, sh->D, qg, groups);
+    const long long longest = std::max(1LL, (sh->max_seq_len + bt - 1) / bt);
+    const long long tiles = groups * longest;
+    // the longest run: an even share of the batch, or what keeps a merge group's pieces within one merge
+    const long long run = std::max(tiles / n, 2 * (longest / 60 + 1)) + 4;
+    if (tiles >= 0x20000000LL || run * bt > (long long)(va::MAX_SPLIT_PAGES - 2) * sh->page_rows) return 0;
+    return (int)n;
+}
+
 bool fused_ok(int groups, int qg, int S) {
     return S <= 64 && groups <= va::TICKET_MAXH && (long long)groups * qg * S <= va::PART_CAP;
 }
 
 int launch_ex(va_fmt fmt, va::DecodeArgs& a, int D, int G, int qg, bool paged, int groups,
               int heads_total, void* stream) {
-    const Lease lease = fused_ok(groups, qg, a.S) ? ticket_slot_for(stream) : Lease{};
+    const bool balanced = a.nwg > 0;
+    const Lease lease = balanced || fused_ok(groups, qg, a.S) ? ticket_slot_for(stream) : Lease{};
     a.ticket_slot = lease.slot;
+    if (lease.slot < 0) a.nwg = 0;
     const bool fused = a.ticket_slot >= 0;
     a.qscale = (float)(1.4426950408889634074 / std::sqrt((double)D));
     hipError_t e = va::launch_decode_ex(kind_of(fmt), D, is_f16(fmt) ? 64 : G, qg, paged, groups, a,
@@ -606,6 +640,13 @@ int va_pick_splits_paged(va_fmt fmt, const va_paged_shape* sh, int* S) {
     if (rc) return rc;
     int qg, nsub, chunk;
     pick_qg(kind_of(fmt), sh->D, sh->Hq / sh->Hkv, &qg, &nsub);
+    const long long groups = (long long)sh->B * sh->Hkv * nsub;
+    const long long n = balanced_wgs(kind_of(fmt), sh, qg, groups, 0);
+    if (n > 0) {                                 // pieces of a balanced launch
+        const long long heads = (long long)sh->B * sh->Hq;
+        *S = (int)(((groups + n) * qg + heads - 1) / heads);
+        return VA_OK;
+    }
     splits_ex(kind_of(fmt), sh->D, qg, sh->B * sh->Hkv * nsub, std::max(1, sh->max_seq_len), 0, S, &chunk);
     // a split may span at most MAX_SPLIT_PAGES pages
     while ((chunk / sh->page_rows) + 2 > va::MAX_SPLIT_PAGES && *S < 0x7FFF) {
@@ -669,6 +710,8 @@ int va_decode_paged(va_fmt fmt, const va_paged_bufs* b, const va_paged_shape* sh
     a.max_pages = sh->max_pages;
     a.page_shift = log2i(sh->page_rows);
     a.num_pages = sh->num_pages;
+    a.nwg = balanced_wgs(kind_of(fmt), sh, qg, groups, S);
+    a.B = sh->B;
     return launch_ex(fmt, a, sh->D, sh->G, qg, true, (int)groups, sh->B * sh->Hq, stream);
 }
 
