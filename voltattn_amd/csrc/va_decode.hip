@@ -236,6 +236,12 @@ int groups_per_cu(int kind, bool tiled) {
     return tiled ? 1 : 8;                 // naive: one position per wave, 32 waves per CU
 }
 
+// q8 and q4 (4-wave groups): H 40, D 128, G 64, L 10007 with one group per CU (S 6)
+// against two (S 12) q8 20.7 -> 18.4 us, q4 14.7 -> 13.1; L 65536 107.5 -> 100.7 and 66.1
+// -> 57.7; H 20, L 20000 20.7 -> 19.8 and 14.7 -> 13.8. f16 is about even (H 40 33.9 ->
+// 32.5, H 24, L 8192 17.1 -> 18.2) and stays at one; two q3 groups do not fit a CU.
+bool two_groups_fit(int kind) { return kind == KQ8 || kind == KQ4; }
+
 template <int KIND, int D, int G>
 static hipError_t launch_one(bool tiled, int H, const DecodeArgs& a, hipStream_t st) {
     const dim3 grid((unsigned)(H * a.S));

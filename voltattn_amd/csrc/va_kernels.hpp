@@ -106,6 +106,10 @@ int ex_groups_per_cu(int kind, int D, int qg);
 // groups per CU of the kind; naive kernels: 8).
 int groups_per_cu(int kind, bool tiled);
 
+// Whether the split rule gives the tiled kernel of `kind` two groups per CU where the
+// heads do not divide the CUs: finer splits even out what the rounding leaves idle.
+bool two_groups_fit(int kind);
+
 // Positions one work-group of the tiled kernel covers per loop iteration;
 // split lengths that are multiples of it leave no partial tile.
 int tile_positions(int kind, bool tiled, int D);

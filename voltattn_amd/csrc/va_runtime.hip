@@ -262,6 +262,15 @@ int cu_count() {
     return n;
 }
 
+// Splits per merge group so that `groups` of them fill `slots` work-group slots: as
+// many as fit in one round. (One more each, which the reference's rule rounds up to,
+// leaves a few work-groups for a second round: H 40, D 128, G 64 on MI355X, S 7 -> 6,
+// L 10007: q3 20.7 -> 13.0 us, f16 41.3 -> 33.9.) Above half the slots rounding down
+// would idle up to half of them, and the groups are many enough to overlap.
+int whole_splits(int slots, int groups) {
+    return std::max(1, 2 * groups <= slots ? slots / groups : (slots + groups - 1) / groups);
+}
+
 } // namespace
 
 extern "C" {
@@ -304,11 +313,16 @@ int va_pick_splits(va_fmt fmt, int H, int L, int D, int* S) {
     // stream a CU at full rate; more splits only lengthen the merge). Naive
     // kernels keep one position per wave in flight, so they need ~8 per CU.
     int per_cu = va::groups_per_cu(kind_of(fmt), tiled_of(fmt));
+    // two where the heads leave more than 1/32 of the CUs idle, once there is work for it
+    // (at 800 to 940 positions per CU q4 loses 0.6 us with them)
+    if (tiled_of(fmt) && va::two_groups_fit(kind_of(fmt)) && H <= cus && H * (cus / H) < cus - cus / 32 &&
+        (long long)H * L >= 1280LL * cus)
+        per_cu = 2;
     // (q3 once took a second work-group per CU on long contexts, while its
     // kernel fit four waves per SIMD. The kernel now holds ~150 VGPRs, one
     // group per CU, and one split per CU measured faster on MI355X (H=32,
     // D=128): L=65536 46.2 -> 42.4 us, L=262144 157.6 -> 156.2 us.)
-    const int target = std::max(1, (per_cu * cus + H - 1) / H);
+    const int target = whole_splits(per_cu * cus, H);
     const int s0     = std::max(1, std::min(tiles, target));
     const int tps    = (tiles + s0 - 1) / s0;               // tiles per split
     *S = std::max(1, (L + tps * tb - 1) / (tps * tb));
@@ -475,7 +489,7 @@ void splits_ex(int kind, int D, int qg, int groups, int max_len, int S_req, int*
     const int tb = va::tile_positions_ex(kind, D);
     const int tiles = std::max(1, (max_len + tb - 1) / tb);
     int s0 = S_req;
-    if (s0 <= 0) s0 = std::max(1, std::min(std::min(tiles, 64), (cus + groups - 1) / groups));
+    if (s0 <= 0) s0 = std::max(1, std::min(std::min(tiles, 64), whole_splits(cus, groups)));
     const int tps = (tiles + s0 - 1) / s0;
     *chunk = tps * tb;
     *S = S_req > 0 ? S_req : std::max(1, (max_len + *chunk - 1) / *chunk);
