@@ -26,6 +26,17 @@ def test_groups_fit_whole_rounds(fmt, L):
         assert Hkv * va.pick_splits_gqa(fmt, 4 * Hkv, Hkv, L, 128) <= CUS
 
 
+@pytest.mark.parametrize("fmt", TILED, ids=lambda f: f.label)
+@pytest.mark.parametrize("B,Hq,Hkv", [(2, 32, 8), (16, 8, 8), (64, 32, 8), (100, 64, 8)])
+@pytest.mark.parametrize("L", [300, 16384, 1 << 20])
+def test_paged_splits_hold_pieces_and_pages(fmt, B, Hq, Hkv, L):
+    """The picked count keeps a split within the pages that a work-group stages (1024), for
+    calls that get no ticket slot, as well as giving the workspace of a balanced launch."""
+    shape = va.PagedShape(B, Hq, Hkv, 128, 32, 64, L // 64 + 1, 1 << 14, L)
+    S = va.pick_splits_paged(fmt, shape)
+    assert S >= 1 and (-(-L // S) + 64) // 64 + 2 <= 1024, S
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", TILED, ids=lambda f: f.label)
 @pytest.mark.parametrize("H,L", [(33, 10300), (40, 8191), (60, 2000)])

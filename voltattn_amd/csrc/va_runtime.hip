@@ -655,13 +655,12 @@ int va_pick_splits_paged(va_fmt fmt, const va_paged_shape* sh, int* S) {
     int qg, nsub, chunk;
     pick_qg(kind_of(fmt), sh->D, sh->Hq / sh->Hkv, &qg, &nsub);
     const long long groups = (long long)sh->B * sh->Hkv * nsub;
+    // Balanced: splits enough for its pieces' partials (the launch takes the splits
+    // themselves where it gets no ticket slot, so they obey the same limits).
     const long long n = balanced_wgs(kind_of(fmt), sh, qg, groups, 0);
-    if (n > 0) {                                 // pieces of a balanced launch
-        const long long heads = (long long)sh->B * sh->Hq;
-        *S = (int)(((groups + n) * qg + heads - 1) / heads);
-        return VA_OK;
-    }
-    splits_ex(kind_of(fmt), sh->D, qg, sh->B * sh->Hkv * nsub, std::max(1, sh->max_seq_len), 0, S, &chunk);
+    const long long heads = (long long)sh->B * sh->Hq;
+    const int want = n > 0 ? (int)(((groups + n) * qg + heads - 1) / heads) : 0;
+    splits_ex(kind_of(fmt), sh->D, qg, sh->B * sh->Hkv * nsub, std::max(1, sh->max_seq_len), want, S, &chunk);
     // a split may span at most MAX_SPLIT_PAGES pages
     while ((chunk / sh->page_rows) + 2 > va::MAX_SPLIT_PAGES && *S < 0x7FFF) {
         splits_ex(kind_of(fmt), sh->D, qg, sh->B * sh->Hkv * nsub, std::max(1, sh->max_seq_len), *S * 2, S, &chunk);
