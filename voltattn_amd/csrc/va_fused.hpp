@@ -273,9 +273,8 @@ __device__ void finish_tagged(const DecodeArgs& a, const Route& rt, const float 
     }
 }
 
-// Counted protocol: every work-group stores its partials as plain fp32 (o[0..D),
-// m, l; PSF floats each, partial (q, s) of merge group mg at (mg*QG + q)*S + s)
-// with device-coherent stores while thread NT-1 takes the merge group's ticket
+// Counted protocol: every work-group stores its partials as plain fp32 (PartStore:
+// the slot's store, or ws for the pieces of a balanced run) with device-coherent stores while thread NT-1 takes the merge group's ticket
 // (word 0 of the group's ticket line), so the stores' round trip overlaps the
 // ticket's. Every thread then waits until its stores (or the atomic) have
 // completed, and after the barrier a work-group that did not complete the

@@ -54,9 +54,9 @@ struct DecodeArgs {
 // atomics to one line serialize at the memory side, and the S arrivals of every
 // group land together. The partials of a fused call live in library memory
 // (PART_CAP partials per slot: PART_STRIDE 64-bit words tagged, PARTF_STRIDE
-// floats plain), not in the caller's ws.
-// Calls with more than TICKET_MAXH merge groups, more than PART_CAP partials or
-// more than 64 splits use the two-pass form.
+// floats plain), not in the caller's ws; a balanced paged call's live in ws.
+// Calls with more than TICKET_MAXH merge groups, or (balanced ones aside) more than
+// PART_CAP partials or 64 splits, use the two-pass form.
 constexpr int TICKET_SLOTS  = 16;
 constexpr int TICKET_MAXH   = 1024;
 constexpr int TICKET_STRIDE = 64;   // uint32 per ticket line (256 bytes)

@@ -43,7 +43,7 @@
 // lazy running maximum per query slot as in decode_tiled (RESCALE_SLACK).
 //
 // Work split, loads and the merge are decode_tiled's: one work-group per
-// (merge group, split), per-wave 32-row tiles double-buffered in registers,
+// (merge group, split), or per run of a balanced paged batch (BAL, va_balance.hpp), per-wave 32-row tiles double-buffered in registers,
 // buffer resources bounded by the split (or per tile for paged caches), and
 // finish_partial for the partials / fused merge.
 #pragma once

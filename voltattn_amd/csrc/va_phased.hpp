@@ -6,7 +6,7 @@
 // the K and V rows of a split read in separate phases. The paged form needs
 // pages of at least one work-group tile (TB rows, a power of two) and splits
 // that start on a tile, so that every tile lies in one page; the host checks
-// both.
+// both. BAL: the items of a balanced run instead of one split (va_balance.hpp).
 //
 // A work-group walks its split in rounds of up to RT work-group tiles. Each
 // round first streams the K rows of its positions (with the K scales): every

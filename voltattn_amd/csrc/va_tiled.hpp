@@ -30,6 +30,9 @@
 // load at or past the split end returns 0 with no memory access (partial
 // tiles, and the prefetch beyond the last tile).
 //
+// Balanced form (BAL, paged only): the work-group walks the items of a run instead of
+// one split (va_balance.hpp).
+//
 // Paged form: rows of sequence b live in pages of 2^page_shift rows, page p
 // holding [hkv][page_rows][row] of the pool; position j of sequence b is row
 // j mod page_rows of page block_table[b][j / page_rows]. Page sizes are
