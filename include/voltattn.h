@@ -281,7 +281,8 @@ typedef struct {
     const uint16_t* sk;            /* K scale pool (quantized formats) */
     const uint16_t* sv;            /* V scale pool */
     const int32_t*  block_table;   /* [B][max_pages] page ids */
-    const int32_t*  seq_lens;      /* [B] positions per sequence (0 .. max_seq_len) */
+    const int32_t*  seq_lens;      /* [B] positions per sequence (0 .. max_seq_len); like the
+                                    * other inputs unchanged until the call has run */
     const uint16_t* q;             /* [B][Hq][D] fp16 */
     uint16_t*       out;           /* [B][Hq][D] fp16 */
     float*          ws;            /* va_ws_bytes(B * Hq, D, S) bytes */
@@ -293,10 +294,14 @@ typedef struct {
  * equal shares of the positions that are there, as many as the S splits' ws
  * holds partials for; otherwise splits are S ranges of ceil(max_seq_len / S)
  * positions (rounded up to the kernel tile), and a sequence shorter than
- * max_seq_len leaves its later splits empty. A sequence of length 0 gives a zero output; a length above
- * max_seq_len, or a page id outside the pool on one of its positions, gives
- * NaN for that sequence's heads. S = 0 picks the split count
- * (va_pick_splits_paged). Asynchronous on `stream`. */
+ * max_seq_len leaves its later splits empty. Equal shares depend on the lengths
+ * of the whole batch, and so do the last bits of a sequence's sums; the same
+ * batch gives the same bits. A length rewritten while the call runs leaves the
+ * outputs undefined, of this call and, where its shares no longer agree on a
+ * merge, of later balanced calls on the stream. A sequence of length 0 gives a
+ * zero output; a length above max_seq_len, or a page id outside the pool on one
+ * of its positions, gives NaN for that sequence's heads. S = 0 picks the split
+ * count (va_pick_splits_paged). Asynchronous on `stream`. */
 int va_decode_paged(va_fmt fmt, const va_paged_bufs* b, const va_paged_shape* shape, int S,
                     void* stream);
 int va_pick_splits_paged(va_fmt fmt, const va_paged_shape* shape, int* S);

@@ -5,6 +5,7 @@
 // that calls the HIP runtime API.
 #include "voltattn.h"
 #include "va_kernels.hpp"
+#include "va_runs.hpp"
 #include "va_slots.hpp"
 
 #include <hip/hip_runtime.h>
@@ -516,6 +517,7 @@ int balanced_wgs(int kind, const va_paged_shape* sh, int qg, long long groups, i
     if (sh->B < 2 || groups > va::TICKET_MAXH) return 0;
     if (groups <= cus && groups * sh->max_seq_len < 2048LL * cus) return 0;
     long long n = va::balanced_groups(kind, sh->D, qg, groups, cus);
+    n = std::min(n, (long long)va::MAX_RUNS);
     if (S > 0) n = std::min(n, (long long)sh->B * sh->Hq * S / qg - groups);
     if (n < cus) return 0;
     const long long bt = va::balanced_tile(kind, sh->D, qg, groups);
