@@ -119,10 +119,9 @@ struct Balance : Runs<COST, MIN_RUN> {
 // End of an item of a balanced run: output if the merge group lies in one run,
 // otherwise a partial and, by the last arrival, the merge.
 template <int D, int NT, int QG, class Bal>
-__device__ __forceinline__ void finish_item(const DecodeArgs& a, const Route& rt, const Bal& w,
+__device__ __forceinline__ void finish_item(int t, const DecodeArgs& a, const Route& rt, const Bal& w,
                                             const float (&M)[QG], const float (&ls)[QG], const float (&acc)[QG]) {
     if (w.pieces == 1) {
-        const int t = (int)threadIdx.x;
         if (t < D) {
 #pragma unroll
             for (int q = 0; q < QG; ++q) {
@@ -134,7 +133,7 @@ __device__ __forceinline__ void finish_item(const DecodeArgs& a, const Route& rt
     }
     constexpr int PSF = D + 2;
     const PartStore ps{a.ws + (size_t)(rt.mg + w.first) * (QG * PSF), QG * PSF, PSF, w.pieces, (int)blockIdx.x - w.first};
-    finish_counted<D, NT, QG>(a, rt, ps, M, ls, acc);
+    finish_counted<D, NT, QG>(t, a, rt, ps, M, ls, acc);
 }
 
 } // namespace va

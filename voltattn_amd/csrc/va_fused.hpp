@@ -274,9 +274,10 @@ __device__ void finish_tagged(const DecodeArgs& a, const Route& rt, const float 
 }
 
 // Counted protocol: every work-group stores its partials as plain fp32 (PartStore:
-// the slot's store, or ws for the pieces of a balanced run) with device-coherent stores while thread NT-1 takes the merge group's ticket
-// (word 0 of the group's ticket line), so the stores' round trip overlaps the
-// ticket's. Every thread then waits until its stores (or the atomic) have
+// the slot's store, or ws for the pieces of a balanced run) with device-coherent
+// stores while thread NT-1 takes the merge group's ticket (word 0 of the group's
+// ticket line), so the stores' round trip overlaps the ticket's. Every thread
+// (t: its index) then waits until its stores (or the atomic) have
 // completed, and after the barrier a work-group that did not complete the
 // ticket counts itself in word 2 of the line. The work-group that completes the
 // ticket merges from its own partials in LDS (its stores go unused), after
@@ -295,11 +296,10 @@ __device__ void finish_tagged(const DecodeArgs& a, const Route& rt, const float 
 // flagged with l = NaN) gives NaN, and so does a count that never completes
 // within the poll bound. Needs S <= 64.
 template <int D, int NT, int QG>
-__device__ void finish_counted(const DecodeArgs& a, const Route& rt, const PartStore& ps, const float (&M)[QG],
+__device__ void finish_counted(int t, const DecodeArgs& a, const Route& rt, const PartStore& ps, const float (&M)[QG],
                                const float (&ls)[QG], const float (&acc)[QG]) {
     constexpr int NW = NT / 64;
     const uint32_t PB = (uint32_t)ps.ss * 4u;    // bytes from one split's partial to the next
-    const int t = (int)threadIdx.x;
     const int S = ps.S, s = ps.s;
     constexpr int WQ = NW / QG;
     static_assert(NW >= QG && NW % QG == 0, "whole waves per query slot");
@@ -488,7 +488,7 @@ __device__ void finish_partial(const DecodeArgs& a, const Route& rt, const float
         static_assert(PSF <= PARTF_STRIDE, "partial store");
         const PartStore ps{g_partf + (size_t)a.ticket_slot * PART_CAP * PARTF_STRIDE + (size_t)rt.mg * QG * S * PSF,
                            PSF, S * PSF, S, s};
-        finish_counted<D, NT, QG>(a, rt, ps, M, ls, acc);
+        finish_counted<D, NT, QG>(t, a, rt, ps, M, ls, acc);
     }
 }
 

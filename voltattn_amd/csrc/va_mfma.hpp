@@ -669,7 +669,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void decode_mfma(De
         acc[q] = t < D ? s_acc[q][t] : 0.f;
     }
     if constexpr (BAL) {
-        finish_item<D, WAVES * 64, QG>(a, rt, bal, M, ls, acc);
+        finish_item<D, WAVES * 64, QG>(tid, a, rt, bal, M, ls, acc);
         bal.advance();
     } else {
         finish_partial<D, WAVES * 64, QG>(a, rt, M, ls, acc, epoch);

@@ -389,8 +389,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
     }
 
     if (BAL && n <= 0) bal.locate();
-    group_finish<D, LP, EPL, WAVES, QG, PAGED>(m, l, o, bad, [&](auto& M, auto& ls, auto& acc) {
-        if constexpr (BAL) finish_item<D, WAVES * 64, QG>(a, rt, bal, M, ls, acc);
+    group_finish<D, LP, EPL, WAVES, QG, PAGED>(tid, m, l, o, bad, [&](auto& M, auto& ls, auto& acc) {
+        if constexpr (BAL) finish_item<D, WAVES * 64, QG>(tid, a, rt, bal, M, ls, acc);
         else finish_partial<D, WAVES * 64, QG>(a, rt, M, ls, acc, epoch);
     });
     if constexpr (BAL) {

@@ -89,16 +89,21 @@ __device__ __forceinline__ void fix_finish(float* o, float s, std::integer_seque
 // uniform, in log2 units; l[q] and o[q][EPL] over the lane's rows, l repeated
 // on the LP lanes of a row) is folded into one partial (M, l, o[D]) per query
 // slot — the slots of a DPP row first, then rows and waves via LDS — and
-// handed to `finish` (finish_partial, or finish_item of a balanced run). A paged tile with a bad page id in any wave
-// (`bad`) marks every partial of the group (l = NaN).
+// handed to `finish` (finish_partial, or finish_item of a balanced run). A paged
+// tile with a bad page id in any wave (`bad`) marks every partial of the group
+// (l = NaN). `t` is the thread; a balanced kernel hands in the value that it made
+// opaque for the item, here and to finish_item: addresses and lane masks derived
+// from threadIdx itself were computed ahead of the item loop and held across it, 10
+// to 16 VGPRs (f16 with two query slots went to scratch: batch of 8 x 16384, Hq 16 /
+// Hkv 8, 91.1 -> 85.4 us without).
 template <int D, int LP, int EPL, int WAVES, int QG, bool PAGED, class Finish>
-__device__ __forceinline__ void group_finish(const float (&m)[QG], float (&l)[QG], float (&o)[QG][EPL], bool bad,
-                                             const Finish& finish) {
+__device__ __forceinline__ void group_finish(int t, const float (&m)[QG], float (&l)[QG], float (&o)[QG][EPL],
+                                             bool bad, const Finish& finish) {
     __shared__ float s_red[QG][WAVES * 4][D + 1];
     __shared__ float s_l[QG][WAVES];
     __shared__ float s_m[QG][WAVES];
-    const int wave = uniform((int)(threadIdx.x >> 6));
-    const int lane = (int)(threadIdx.x & 63);
+    const int wave = uniform(t >> 6);
+    const int lane = t & 63;
     const int sl   = lane % LP;
 #pragma unroll
     for (int q = 0; q < QG; ++q) {
@@ -140,7 +145,6 @@ __device__ __forceinline__ void group_finish(const float (&m)[QG], float (&l)[QG
     bool any_bad = false;
     if constexpr (PAGED) any_bad = __syncthreads_or(bad);
     else __syncthreads();
-    const int t = (int)threadIdx.x;
     float M[QG], acc[QG], ls[QG];
     if constexpr (QG < 4) {
         // threads t < D fold every query slot of dimension t (measured faster
@@ -561,8 +565,8 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void decode_tiled(
     }
 
     if (BAL && n <= 0) bal.locate();
-    group_finish<D, LP, EPL, WAVES, QG, PAGED>(m, l, o, bad, [&](auto& M, auto& ls, auto& acc) {
-        if constexpr (BAL) finish_item<D, WAVES * 64, QG>(a, rt, bal, M, ls, acc);
+    group_finish<D, LP, EPL, WAVES, QG, PAGED>(tid, m, l, o, bad, [&](auto& M, auto& ls, auto& acc) {
+        if constexpr (BAL) finish_item<D, WAVES * 64, QG>(tid, a, rt, bal, M, ls, acc);
         else finish_partial<D, WAVES * 64, QG>(a, rt, M, ls, acc, epoch);
     });
     if constexpr (BAL) {
