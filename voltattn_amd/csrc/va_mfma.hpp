@@ -277,9 +277,10 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void decode_mfma(De
                 if (rows > 0) page = uniform(s_page[(pos >> a.page_shift) - p0]);
                 const bool ok = page >= 0 && page < a.num_pages;
                 bad = bad || (rows > 0 && !ok);
-                const uint32_t nrow = ok ? (uint32_t)rows : 0u;
-                const size_t row = ((size_t)(ok ? page : 0) * a.hkv + hk) * ((size_t)1 << a.page_shift) +
-                                   (size_t)(pos & ((1 << a.page_shift) - 1));
+                // every descriptor field scalar: one in a VGPR would make each load a loop over lanes
+                const uint32_t nrow = sgpr(ok ? (uint32_t)rows : 0u);
+                const size_t row = uniform64(((size_t)(ok ? page : 0) * a.hkv + hk) * ((size_t)1 << a.page_shift) +
+                                             (size_t)(pos & ((1 << a.page_shift) - 1)));
                 tk  = make_rsrc(a.k + row * ROWB, nrow * ROWB);
                 tv  = make_rsrc(a.v + row * ROWB, nrow * ROWB);
                 tsk = make_rsrc(a.sk + row * NG, nrow * NG * 2);
