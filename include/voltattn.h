@@ -298,7 +298,7 @@ typedef struct {
  * of the whole batch, and so do the last bits of a sequence's sums; the same
  * batch gives the same bits. A length rewritten while the call runs leaves the
  * outputs undefined, of this call and, where its shares no longer agree on a
- * merge, of later balanced calls on the stream. A sequence of length 0 gives a
+ * merge, of later calls on the stream. A sequence of length 0 gives a
  * zero output; a length above max_seq_len, or a page id outside the pool on one
  * of its positions, gives NaN for that sequence's heads. S = 0 picks the split
  * count (va_pick_splits_paged). Asynchronous on `stream`. */

@@ -87,6 +87,29 @@ static int check_batch(const std::vector<int>& tiles, int G, int nwg) {
     return most;
 }
 
+// Equal sequences: every merge group in 2^shift pieces, piece s in work-group (mg << shift) + s.
+static void check_even(int t, int shift, int G, int B, int nwg) {
+    va::Runs<1, 1> r;
+    const int P = 1 << shift;
+    int to = 0;
+    for (int w = 0; w < nwg; ++w) {
+        r.plan_even(t, shift, w, B, G);
+        if (w >= B * G * P) {
+            CHECK(!r.next());
+            continue;
+        }
+        CHECK(r.next());
+        r.locate();
+        CHECK(r.b * G + r.g == w / P && r.g >= 0 && r.g < G && r.first == w / P * P && r.pieces == P);
+        if (w % P == 0) to = 0;
+        CHECK(r.t0 == to && r.cnt >= 1 && r.cnt <= t / P + 1);
+        to += r.cnt;
+        if (w % P == P - 1) CHECK(to == t);
+        if (r.pass()) r.ub = t;
+        CHECK(!r.next());                                    // one item each
+    }
+}
+
 template <int COST>
 static void random_batches(unsigned seed) {
     using R = va::Runs<COST, COST>;
@@ -133,6 +156,10 @@ int main(int argc, char** argv) {
     int reached = 0;
     for (int t = 50; t < 400; ++t) reached = std::max(reached, check_batch<va::Runs<1, 1>>({t, 1, 1, 3}, 2, 512));
     CHECK(reached == va::MAX_PIECES || reached == va::MAX_PIECES - 1);
+    for (int shift = 0; shift <= 6; ++shift)
+        for (int t : {1 << shift, (1 << shift) + 1, 3 << shift, 1000, 1 << 20})
+            for (int G : {1, 2, 3, 8, 12})
+                if (t >= 1 << shift) check_even(t, shift, G, 512 / (G << shift), 512);
     std::printf("runs: ok\n");
     return 0;
 }

@@ -16,6 +16,13 @@
 // lies at slot mg + w, which no other piece shares (the next merge group starts at
 // work-group w or later), so nwg + (merge groups) slots are enough.
 //
+// Equal lengths (DecodeArgs::even): every merge group in the same power of two of
+// pieces, as static splits would be, found without the plan's divisions and scans. With
+// one query slot such pieces are merged by the tagged protocol in the slot's store.
+// Measured on MI355X, 8 x 16384, D 128, Hq = Hkv = 8, by the plan -> so (static splits):
+// q8 46.5 -> 45.9 us (44.6), f16 82.3 -> 79.0 (78.4); 32 x 4096 46.7 -> 44.5 (44.6) and
+// 82.1 -> 77.1 (77.8); Hq 32 / Hkv 8, 8 x 16384: q8 51.1 -> 49.8 (51.7), q4 37.4 -> 36.1.
+//
 // Every wave walks the plan by itself from seq_lens: one scan over the lengths
 // finds the run's first item, then one length per further sequence. All of it is
 // wave-uniform (va_runs.hpp has the arithmetic).
@@ -54,13 +61,14 @@ __device__ __forceinline__ int wave_scan_max(int x) {           // x >= 0; lane 
     return x;
 }
 
-template <int BT, int COST, int MIN_RUN>
+template <int BT, int COST, int MIN_RUN, int QG>
 struct Balance : Runs<COST, MIN_RUN> {
     using R = Runs<COST, MIN_RUN>;
-    using R::at, R::end, R::base, R::b, R::ub, R::cost;
+    using R::at, R::end, R::base, R::b, R::g, R::ub, R::cost;
     const DecodeArgs& a;
     int len;                // the next item's sequence: its recorded length
     int ahead;              // the sequence after it
+    unsigned epoch;         // equal sequences, tagged protocol (QG = 1): the merge group's, read with the lengths
 
     __device__ __forceinline__ int cap() const { return min(a.L, a.max_pages << a.page_shift); }
     // An invalid length is walked as far as it may be read (its output becomes NaN).
@@ -72,6 +80,20 @@ struct Balance : Runs<COST, MIN_RUN> {
         const int G = a.hkv * a.nsub;
         // lengths 64 at a time; the first 64 stay for the search
         int x = a.seq_lens[min(lane, a.B - 1)];
+        epoch = 0u;
+        if (a.even >= 0) {
+            const int x0 = __builtin_amdgcn_readfirstlane(x), t0 = tiles(x0);
+            epoch = read_epoch<QG>(a, min((int)blockIdx.x >> a.even, a.B * G - 1));
+            bool even = t0 >> a.even > 0 && __builtin_amdgcn_ballot_w64(x != x0) == 0;
+            for (int c = 64; c < a.B && even; c += 64)
+                even = __builtin_amdgcn_ballot_w64(a.seq_lens[min(c + lane, a.B - 1)] != x0) == 0;
+            if (even) {
+                R::plan_even(t0, a.even, (int)blockIdx.x, a.B, G);
+                len = ahead = x0;
+                asm volatile("");                            // keeps the two paths' stores apart (va_runs.hpp)
+                return;
+            }
+        }
         int t = lane < a.B ? tiles(x) : 0, p = wave_scan(t);
         int sum = __builtin_amdgcn_readlane(p, 63);
         int most = __builtin_amdgcn_readlane(wave_scan_max(t), 63);
@@ -107,6 +129,8 @@ struct Balance : Runs<COST, MIN_RUN> {
         ahead = a.seq_lens[min(b + 1, a.B - 1)];
     }
 
+    __device__ __forceinline__ bool even() const { return R::n == 0; }
+
     // Past the current item: it ended its merge group or the run.
     __device__ __forceinline__ void advance() {
         if (!R::pass()) return;
@@ -120,7 +144,8 @@ struct Balance : Runs<COST, MIN_RUN> {
 // otherwise a partial and, by the last arrival, the merge.
 template <int D, int NT, int QG, class Bal>
 __device__ __forceinline__ void finish_item(int t, const DecodeArgs& a, const Route& rt, const Bal& w,
-                                            const float (&M)[QG], const float (&ls)[QG], const float (&acc)[QG]) {
+                                            const float (&M)[QG], const float (&ls)[QG], const float (&acc)[QG],
+                                            unsigned epoch) {
     if (w.pieces == 1) {
         if (t < D) {
 #pragma unroll
@@ -130,6 +155,15 @@ __device__ __forceinline__ void finish_item(int t, const DecodeArgs& a, const Ro
             }
         }
         return;
+    }
+    if constexpr (QG == 1) {
+        if (w.even()) {                          // splits like any others: their protocol is the faster one
+            DecodeArgs e = a;
+            e.S = w.pieces;
+            const Route r{rt.mg, (int)blockIdx.x - w.first, rt.nq, rt.oh0};
+            finish_partial<D, NT, QG>(e, r, M, ls, acc, epoch);
+            return;
+        }
     }
     constexpr int PSF = D + 2;
     const PartStore ps{a.ws + (size_t)(rt.mg + w.first) * (QG * PSF), QG * PSF, PSF, w.pieces, (int)blockIdx.x - w.first};

@@ -36,6 +36,7 @@ struct DecodeArgs {
     // work-group per (merge group, split). Its partials go to ws, its merge needs a ticket slot.
     int   nwg;
     int   B;                // sequences in the batch
+    int   even;             // equal sequences: each merge group in 2^even pieces, one to a work-group; -1: by the plan
 };
 
 // Launch of the tiled decode kernel: the leading scalar arguments (preloaded
@@ -99,6 +100,8 @@ int tile_positions_ex(int kind, int D);
 // groups on `cus` CUs, and the positions of its tiles.
 int balanced_groups(int kind, int D, int qg, long long groups, int cus);
 int balanced_tile(int kind, int D, int qg, long long groups);
+// Those of its nwg work-groups that sequences of equal length are dealt to.
+int balanced_even(int kind, int qg, int nwg, int cus);
 // Work-groups per CU the grouped/paged launch of (kind, QG) is built for.
 int ex_groups_per_cu(int kind, int D, int qg);
 

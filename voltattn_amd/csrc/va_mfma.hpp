@@ -190,7 +190,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void decode_mfma(De
     __shared__ int   s_prog[WAVES];                         // tile pair each wave is on (issue priority)
 
     static_assert(!BAL || PAGED, "balanced runs: paged batches");
-    Balance<TB, 256 / TB, 256 / TB> bal(BAL, a);
+    Balance<TB, 256 / TB, 256 / TB, QG> bal(BAL, a);
     const int wave = uniform((int)(threadIdx.x >> 6));
 
     do {
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void decode_mfma(De
     }
     rt.nq  = min(QG, a.qgroup - sub * QG);
     rt.oh0 = (b * a.hkv + hk) * a.qgroup + sub * QG;
-    const unsigned epoch = read_epoch<QG>(a, rt.mg);
+    const unsigned epoch = BAL ? bal.epoch : read_epoch<QG>(a, rt.mg);
 
     int L = a.L;
     bool bad = false;
@@ -670,7 +670,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 4 ? 2 : 1) void decode_mfma(De
         acc[q] = t < D ? s_acc[q][t] : 0.f;
     }
     if constexpr (BAL) {
-        finish_item<D, WAVES * 64, QG>(tid, a, rt, bal, M, ls, acc);
+        finish_item<D, WAVES * 64, QG>(tid, a, rt, bal, M, ls, acc, epoch);
         bal.advance();
     } else {
         finish_partial<D, WAVES * 64, QG>(a, rt, M, ls, acc, epoch);

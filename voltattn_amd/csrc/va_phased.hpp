@@ -84,7 +84,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
 
     static_assert(!BAL || PAGED, "balanced runs: paged batches");
     constexpr int BT = balance_tile(TB);
-    Balance<BT, 256 / BT, 256 / BT> bal(BAL, a);
+    Balance<BT, 256 / BT, 256 / BT, QG> bal(BAL, a);
     do {
     if (BAL && !bal.next()) return;
     // work-group -> (KV head hk, query sub-group, split s), or the next item of a balanced run
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
         rt.nq  = min(QG, a.qgroup - sub * QG);
         rt.oh0 = hk * a.qgroup + sub * QG;
     }
-    const unsigned epoch = BAL ? 0u : read_epoch<QG>(a, rt.mg);
+    const unsigned epoch = BAL ? bal.epoch : read_epoch<QG>(a, rt.mg);
     int tid = (int)threadIdx.x;
     if constexpr (BAL) asm volatile("" : "+v"(tid));   // per-lane values are not carried from item to item
     const int wave = uniform(tid >> 6);
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_phased(
 
     if (BAL && n <= 0) bal.locate();
     group_finish<D, LP, EPL, WAVES, QG, PAGED>(tid, m, l, o, bad, [&](auto& M, auto& ls, auto& acc) {
-        if constexpr (BAL) finish_item<D, WAVES * 64, QG>(tid, a, rt, bal, M, ls, acc);
+        if constexpr (BAL) finish_item<D, WAVES * 64, QG>(tid, a, rt, bal, M, ls, acc, epoch);
         else finish_partial<D, WAVES * 64, QG>(a, rt, M, ls, acc, epoch);
     });
     if constexpr (BAL) {

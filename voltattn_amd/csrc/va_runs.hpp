@@ -97,11 +97,38 @@ struct Runs {
         at += u1 - u0;
         return true;
     }
+    // Sequences of t >= 2^shift tiles each, every merge group in 2^shift pieces of a
+    // work-group each: what plan() comes to where equal sequences fill the work-groups,
+    // without its divisions. Work-groups past the last merge group have no item.
+    // (Straight-line code: stores to other members on other paths would be joined through a
+    // pointer, and the whole plan kept in scratch memory.)
+    VA_RUNS_FN void plan_even(int t, int shift, int w, int B_, int G_) {
+        const int mg = w >> shift, s = w & ((1 << shift) - 1);
+        const int to = (int)(((int64_t)t * (s + 1)) >> shift);
+        B = B_;
+        G = G_;
+        cost = 0;
+        base = 0;
+        n = 0;                                               // first and pieces are known: locate() leaves them
+        b = (int)((uint32_t)mg / (uint32_t)G_);
+        g = mg - b * G_;
+        ub = t;
+        u0 = (int)(((int64_t)t * s) >> shift);
+        at = 0;
+        end = mg < B_ * G_ ? to - u0 : 0;
+        first = mg << shift;
+        pieces = 1 << shift;
+    }
     // Where the merge group of the current item starts, and its pieces.
     VA_RUNS_FN void locate() {
-        const int gs = base * G + g * ub;                    // the merge group's first unit
-        first = run_of(gs + cost);
-        pieces = run_of(gs + ub - 1) - first + 1;
+        int w = first, k = pieces;
+        if (n > 0) {
+            const int gs = base * G + g * ub;                // the merge group's first unit
+            w = run_of(gs + cost);
+            k = run_of(gs + ub - 1) - w + 1;
+        }
+        first = w;
+        pieces = k;
     }
     // Past the current item, which ended its merge group or the run; true if it was the
     // sequence's last merge group: the caller then sets ub.

@@ -529,6 +529,18 @@ int balanced_wgs(int kind, const va_paged_shape* sh, int qg, long long groups, i
     return (int)n;
 }
 
+// DecodeArgs::even of a balanced launch of nwg work-groups.
+int even_pieces(int kind, const va_paged_shape* sh, int qg, long long groups, int nwg) {
+    if (nwg <= 0) return -1;
+    const int wgs = va::balanced_even(kind, qg, nwg, cu_count());
+    const long long pieces = wgs / groups;
+    if (pieces < 1 || groups * pieces != wgs || (pieces & (pieces - 1)) != 0 || pieces > va::MAX_PIECES) return -1;
+    const long long bt = va::balanced_tile(kind, sh->D, qg, groups);
+    const long long longest = std::max(1LL, (sh->max_seq_len + bt - 1) / bt);
+    if ((longest / pieces + 1) * bt > (long long)(va::MAX_SPLIT_PAGES - 2) * sh->page_rows) return -1;
+    return log2i((int)pieces);
+}
+
 bool fused_ok(int groups, int qg, int S) {
     return S <= 64 && groups <= va::TICKET_MAXH && (long long)groups * qg * S <= va::PART_CAP;
 }
@@ -727,6 +739,7 @@ int va_decode_paged(va_fmt fmt, const va_paged_bufs* b, const va_paged_shape* sh
     a.num_pages = sh->num_pages;
     a.nwg = balanced_wgs(kind_of(fmt), sh, qg, groups, S);
     a.B = sh->B;
+    a.even = even_pieces(kind_of(fmt), sh, qg, groups, a.nwg);
     return launch_ex(fmt, a, sh->D, sh->G, qg, true, (int)groups, sh->B * sh->Hq, stream);
 }
 

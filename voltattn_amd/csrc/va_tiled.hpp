@@ -244,7 +244,7 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void decode_tiled(
 
     static_assert(!BAL || PAGED, "balanced runs: paged batches");
     constexpr int BT = balance_tile(TB);
-    Balance<BT, 256 / BT, 256 / BT> bal(BAL, a);
+    Balance<BT, 256 / BT, 256 / BT, QG> bal(BAL, a);
     do {
     if (BAL && !bal.next()) return;
     // ---- work-group -> (sequence b, KV head hk, query sub-group, split s), or
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void decode_tiled(
         rt.nq  = min(QG, a.qgroup - sub * QG);
         rt.oh0 = (b * a.hkv + hk) * a.qgroup + sub * QG;
     }
-    const unsigned epoch = BAL ? 0u : read_epoch<QG>(a, rt.mg);
+    const unsigned epoch = BAL ? bal.epoch : read_epoch<QG>(a, rt.mg);
     int tid = (int)threadIdx.x;
     if constexpr (BAL) asm volatile("" : "+v"(tid));   // per-lane values are not carried from item to item
     const int wave = uniform(tid >> 6);
@@ -567,7 +567,7 @@ __global__ __launch_bounds__(WAVES * 64, MINB) void decode_tiled(
 
     if (BAL && n <= 0) bal.locate();
     group_finish<D, LP, EPL, WAVES, QG, PAGED>(tid, m, l, o, bad, [&](auto& M, auto& ls, auto& acc) {
-        if constexpr (BAL) finish_item<D, WAVES * 64, QG>(tid, a, rt, bal, M, ls, acc);
+        if constexpr (BAL) finish_item<D, WAVES * 64, QG>(tid, a, rt, bal, M, ls, acc, epoch);
         else finish_partial<D, WAVES * 64, QG>(a, rt, M, ls, acc, epoch);
     });
     if constexpr (BAL) {
