@@ -131,7 +131,7 @@ static int max_tile() {
 // 20.8, f16 32.9 -> 31.1; batch of 16 up to 8192 q8 17.4 -> 15.4), one where fewer merge
 // groups meet longer items (q4 at D 128 16.5 against 18.0, D 64 q8 13.5 against 15.1).
 // Grouped f16 and q3 at D = 64 (8-wave groups): one (f16 26.1 against 34.1).
-static int bal_waves(int kind, long long groups) { return kind != KQ8 && groups > 256 ? 4 : 8; }
+int balanced_waves(int kind, long long groups, int cus) { return kind != KQ8 && groups > cus ? 4 : 8; }
 
 template <int KIND, int D>
 static int bal_tile(int qg) {
@@ -139,13 +139,13 @@ static int bal_tile(int qg) {
 }
 
 int balanced_groups(int kind, int D, int qg, long long groups, int cus) {
-    if (mfma_form(kind, D, qg)) return cus * 8 / bal_waves(kind, groups);
+    if (mfma_form(kind, D, qg)) return cus * 8 / balanced_waves(kind, groups, cus);
     const bool two = qg == 1 && (groups >= cus || (D == 128 && kind != KQ4));
     return two ? 2 * cus : cus;
 }
 
-int balanced_tile(int kind, int D, int qg, long long groups) {
-    if (mfma_form(kind, D, qg)) return 32 * bal_waves(kind, groups);
+int balanced_tile(int kind, int D, int qg, long long groups, int cus) {
+    if (mfma_form(kind, D, qg)) return 32 * balanced_waves(kind, groups, cus);
     switch (kind) {
         case KF16: return D == 128 ? bal_tile<KF16, 128>(qg) : bal_tile<KF16, 64>(qg);
         case KQ8:  return D == 128 ? bal_tile<KQ8, 128>(qg) : bal_tile<KQ8, 64>(qg);
@@ -158,7 +158,7 @@ int balanced_tile(int kind, int D, int qg, long long groups) {
 // 16384, Hq = Hkv = 8: q3 36.4 -> 26.2 us).
 int balanced_even(int kind, int qg, int nwg, int cus) {
     const bool two = qg == 1 && (kind == KQ4 || kind == KQ3);
-    return two || cus <= 0 ? nwg : std::min(nwg, cus);
+    return two ? nwg : std::min(nwg, cus);
 }
 
 int tile_positions_ex(int kind, int D) {
@@ -222,12 +222,15 @@ static hipError_t launch_ex(int groups, const DecodeArgs& a, hipStream_t st) {
     } else if constexpr (mfma_kind_c<KIND, D> && QG >= 2) {
         if constexpr (PAGED) {
             if (a.nwg > 0) {
-                if (bal_waves(KIND, groups) == 4)
-                    hipLaunchKernelGGL((decode_mfma<KIND, D, G, 4, QG, true, true>), dim3((unsigned)a.nwg), dim3(256), 0,
-                                       st, a);
-                else
-                    hipLaunchKernelGGL((decode_mfma<KIND, D, G, 8, QG, true, true>), dim3((unsigned)a.nwg), dim3(512), 0,
-                                       st, a);
+                if constexpr (KIND != KQ8) {                 // q8 has eight (balanced_waves)
+                    if (a.waves == 4) {
+                        hipLaunchKernelGGL((decode_mfma<KIND, D, G, 4, QG, true, true>), dim3((unsigned)a.nwg), dim3(256),
+                                           0, st, a);
+                        return hipGetLastError();
+                    }
+                }
+                hipLaunchKernelGGL((decode_mfma<KIND, D, G, 8, QG, true, true>), dim3((unsigned)a.nwg), dim3(512), 0, st,
+                                   a);
                 return hipGetLastError();
             }
         }

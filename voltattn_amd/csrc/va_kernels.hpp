@@ -35,6 +35,7 @@ struct DecodeArgs {
     // balanced paged form (va_balance.hpp): work-groups that share the batch's tiles; 0: one
     // work-group per (merge group, split). Its partials go to ws, its merge needs a ticket slot.
     int   nwg;
+    int   waves;            // per work-group, matrix-core form
     int   B;                // sequences in the batch
     int   even;             // equal sequences: each merge group in 2^even pieces, one to a work-group; -1: by the plan
 };
@@ -99,7 +100,9 @@ int tile_positions_ex(int kind, int D);
 // Work-groups of a balanced paged launch (DecodeArgs::nwg) over `groups` merge
 // groups on `cus` CUs, and the positions of its tiles.
 int balanced_groups(int kind, int D, int qg, long long groups, int cus);
-int balanced_tile(int kind, int D, int qg, long long groups);
+int balanced_tile(int kind, int D, int qg, long long groups, int cus);
+// Waves per work-group of its matrix-core form.
+int balanced_waves(int kind, long long groups, int cus);
 // Those of its nwg work-groups that sequences of equal length are dealt to.
 int balanced_even(int kind, int qg, int nwg, int cus);
 // Work-groups per CU the grouped/paged launch of (kind, QG) is built for.

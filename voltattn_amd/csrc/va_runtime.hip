@@ -263,6 +263,12 @@ int cu_count() {
     return n;
 }
 
+// Without a device: MI355X's.
+int cus_or_default() {
+    const int n = cu_count();
+    return n > 0 ? n : 256;
+}
+
 // Splits per merge group so that `groups` of them fill `slots` work-group slots: as
 // many as fit in one round. (One more each, which the reference's rule rounds up to,
 // leaves a few work-groups for a second round: H 40, D 128, G 64 on MI355X, S 7 -> 6,
@@ -306,8 +312,7 @@ int va_pick_splits(va_fmt fmt, int H, int L, int D, int* S) {
     if (!S) return fail(VA_ENULL, "S is NULL");
     if (!valid_fmt(fmt) || H < 1 || L < 1 || (D != 64 && D != 128))
         return fail(VA_EINVAL, "invalid arguments to va_pick_splits");
-    int cus = cu_count();
-    if (cus <= 0) cus = 256;
+    const int cus = cus_or_default();
     const int tb    = va::tile_positions(kind_of(fmt), tiled_of(fmt), D);
     const int tiles = (L + tb - 1) / tb;
     // Tiled kernels: the kind's configured groups per CU (one or two groups
@@ -484,9 +489,7 @@ void pick_qg(int kind, int D, int qgroup, int* qg, int* nsub) {
 // groups), splits of whole kernel tiles, at most 64 splits (the fused merge's
 // limit). S_req > 0 fixes S.
 void splits_ex(int kind, int D, int qg, int groups, int max_len, int S_req, int* S, int* chunk) {
-    int cus = cu_count();
-    if (cus <= 0) cus = 256;
-    cus *= va::ex_groups_per_cu(kind, D, qg);
+    const int cus = cus_or_default() * va::ex_groups_per_cu(kind, D, qg);
     const int tb = va::tile_positions_ex(kind, D);
     const int tiles = std::max(1, (max_len + tb - 1) / tb);
     int s0 = S_req;
@@ -511,16 +514,14 @@ void splits_ex(int kind, int D, int qg, int groups, int max_len, int S_req, int*
 // Also 0: one sequence (its length is what the splits are made for), more merge groups
 // than ticket lines, a run that could span more pages than a work-group stages, or a
 // workspace of S splits (S = 0: any) too small for the pieces of one run per CU.
-int balanced_wgs(int kind, const va_paged_shape* sh, int qg, long long groups, int S) {
-    int cus = cu_count();
-    if (cus <= 0) cus = 256;
+int balanced_wgs(int kind, const va_paged_shape* sh, int qg, long long groups, int S, int cus) {
     if (sh->B < 2 || groups > va::TICKET_MAXH) return 0;
     if (groups <= cus && groups * sh->max_seq_len < 2048LL * cus) return 0;
     long long n = va::balanced_groups(kind, sh->D, qg, groups, cus);
     n = std::min(n, (long long)va::MAX_RUNS);
     if (S > 0) n = std::min(n, (long long)sh->B * sh->Hq * S / qg - groups);
     if (n < cus) return 0;
-    const long long bt = va::balanced_tile(kind, sh->D, qg, groups);
+    const long long bt = va::balanced_tile(kind, sh->D, qg, groups, cus);
     const long long longest = std::max(1LL, (sh->max_seq_len + bt - 1) / bt);
     const long long tiles = groups * longest;
     // the longest run: an even share of the batch, or what keeps a merge group's pieces within one merge
@@ -530,12 +531,12 @@ int balanced_wgs(int kind, const va_paged_shape* sh, int qg, long long groups, i
 }
 
 // DecodeArgs::even of a balanced launch of nwg work-groups.
-int even_pieces(int kind, const va_paged_shape* sh, int qg, long long groups, int nwg) {
+int even_pieces(int kind, const va_paged_shape* sh, int qg, long long groups, int nwg, int cus) {
     if (nwg <= 0) return -1;
-    const int wgs = va::balanced_even(kind, qg, nwg, cu_count());
+    const int wgs = va::balanced_even(kind, qg, nwg, cus);
     const long long pieces = wgs / groups;
     if (pieces < 1 || groups * pieces != wgs || (pieces & (pieces - 1)) != 0 || pieces > va::MAX_PIECES) return -1;
-    const long long bt = va::balanced_tile(kind, sh->D, qg, groups);
+    const long long bt = va::balanced_tile(kind, sh->D, qg, groups, cus);
     const long long longest = std::max(1LL, (sh->max_seq_len + bt - 1) / bt);
     if ((longest / pieces + 1) * bt > (long long)(va::MAX_SPLIT_PAGES - 2) * sh->page_rows) return -1;
     return log2i((int)pieces);
@@ -671,7 +672,7 @@ int va_pick_splits_paged(va_fmt fmt, const va_paged_shape* sh, int* S) {
     const long long groups = (long long)sh->B * sh->Hkv * nsub;
     // Balanced: splits enough for its pieces' partials (the launch takes the splits
     // themselves where it gets no ticket slot, so they obey the same limits).
-    const long long n = balanced_wgs(kind_of(fmt), sh, qg, groups, 0);
+    const long long n = balanced_wgs(kind_of(fmt), sh, qg, groups, 0, cus_or_default());
     const long long heads = (long long)sh->B * sh->Hq;
     const int want = n > 0 ? (int)(((groups + n) * qg + heads - 1) / heads) : 0;
     splits_ex(kind_of(fmt), sh->D, qg, sh->B * sh->Hkv * nsub, std::max(1, sh->max_seq_len), want, S, &chunk);
@@ -737,9 +738,11 @@ int va_decode_paged(va_fmt fmt, const va_paged_bufs* b, const va_paged_shape* sh
     a.max_pages = sh->max_pages;
     a.page_shift = log2i(sh->page_rows);
     a.num_pages = sh->num_pages;
-    a.nwg = balanced_wgs(kind_of(fmt), sh, qg, groups, S);
+    const int cus = cus_or_default();
+    a.nwg = balanced_wgs(kind_of(fmt), sh, qg, groups, S, cus);
+    a.waves = va::balanced_waves(kind_of(fmt), groups, cus);
     a.B = sh->B;
-    a.even = even_pieces(kind_of(fmt), sh, qg, groups, a.nwg);
+    a.even = even_pieces(kind_of(fmt), sh, qg, groups, a.nwg, cus);
     return launch_ex(fmt, a, sh->D, sh->G, qg, true, (int)groups, sh->B * sh->Hq, stream);
 }
 
