@@ -13,6 +13,9 @@ from oracle import batch
 import voltattn_amd as va
 
 
+UNWRITTEN = 0x7FA5A5A5                  # a NaN that no kernel produces
+
+
 def f16(x) -> np.ndarray:
     return np.asarray(x, np.float32).astype(np.float16).view(np.uint16)
 
@@ -88,12 +91,15 @@ class PagedBatch:
         self.bufs.append(d)
         return d.ptr
 
-    def run(self, S: int = 0, seq_lens=None, table=None) -> np.ndarray:
+    def run(self, S: int = 0, seq_lens=None, table=None, stream=None) -> np.ndarray:
+        """One decode; self.ws_floats is then the number of floats it wrote to ws: all of the
+        splits' in the two-pass form, those of the cut merge groups' pieces in a balanced
+        launch, none where the merge group's partials stay in library memory."""
         B = len(self.lens)
         quant = self.kspool is not None
         Sx = S or va.pick_splits_paged(self.fmt, self.shape)
         out = va.DeviceBuffer(B * self.Hq * self.D * 2)
-        ws = va.DeviceBuffer(va.ws_bytes(B * self.Hq, self.D, Sx))
+        ws = va.DeviceBuffer.from_array(np.full(va.ws_bytes(B * self.Hq, self.D, Sx) // 4, UNWRITTEN, np.uint32))
         self.bufs += [out, ws]
         b = va.PagedBufs(
             K=self._dev(self.kpool), V=self._dev(self.vpool),
@@ -101,8 +107,9 @@ class PagedBatch:
             block_table=self._dev(self.table if table is None else table),
             seq_lens=self._dev(self.seq_lens if seq_lens is None else np.asarray(seq_lens, np.int32)),
             q=self._dev(self.q), out=out.ptr, ws=ws.ptr)
-        va.decode_paged(self.fmt, b, self.shape, S)
+        va.decode_paged(self.fmt, b, self.shape, S, stream=stream)
         va.sync()
+        self.ws_floats = int(np.count_nonzero(ws.download(np.uint32) != UNWRITTEN))
         return out.download(np.uint16).view(np.float16).astype(np.float32).reshape(B, self.Hq, self.D)
 
     def free(self):

@@ -2,8 +2,9 @@
 // g++ and run by tests/test_runs.py.
 //
 //   test_runs                          checks random batches, prints "runs: ok"
-//   test_runs MIN NWG G TILES...       prints "runs N pieces P" of one batch: its runs
-//                                      and the most pieces of any merge group
+//   test_runs MIN NWG G TILES...       prints "runs N pieces P partials Q" of one batch: its
+//                                      runs, the most pieces of any merge group and the
+//                                      pieces of all merge groups that are cut
 #include "va_runs.hpp"
 
 #include <algorithm>
@@ -137,16 +138,16 @@ int main(int argc, char** argv) {
         const int min_run = std::atoi(argv[1]), nwg = std::atoi(argv[2]), G = std::atoi(argv[3]);
         std::vector<int> tiles;
         for (int i = 4; i < argc; ++i) tiles.push_back(std::atoi(argv[i]));
-        int most = 0, n = 0;
+        int most = 0, n = 0, cut = 0;
         const auto one = [&](auto r) {
             most = check_batch<decltype(r)>(tiles, G, nwg);
-            walk(r, tiles, G, nwg);
+            for (const Item& x : walk(r, tiles, G, nwg)) cut += x.pieces > 1;
             n = r.n;
         };
         if (min_run == 2) one(va::Runs<2, 2>{});
         else if (min_run == 1) one(va::Runs<1, 1>{});
         else one(va::Runs<0, 0>{});
-        std::printf("runs %d pieces %d\n", n, most);
+        std::printf("runs %d pieces %d partials %d\n", n, most, cut);
         return 0;
     }
     random_batches<2>(1);

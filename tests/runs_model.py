@@ -23,10 +23,9 @@ def run(*args):
     return subprocess.run([_exe()[1], *map(str, args)], capture_output=True, text=True, timeout=120)
 
 
-def plan(lens, tile: int, groups: int, wgs: int) -> tuple[int, int]:
-    """(runs, most pieces of a merge group) of a batch: `tile` positions per tile of the
-    plan, `groups` merge groups per sequence, `wgs` work-groups."""
+def plan(lens, tile: int, groups: int, wgs: int) -> tuple[int, int, int]:
+    """(runs, most pieces of a merge group, pieces of all cut merge groups) of a batch: `tile`
+    positions per tile of the plan, `groups` merge groups per sequence, `wgs` work-groups."""
     r = run(256 // tile, wgs, groups, *(max(1, -(-L // tile)) for L in lens))
     assert r.returncode == 0, r.stderr
-    _, n, _, pieces = r.stdout.split()
-    return int(n), int(pieces)
+    return tuple(int(x) for x in r.stdout.split()[1::2])

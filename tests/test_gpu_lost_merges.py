@@ -10,6 +10,7 @@ kernel still exits normally. Checked in one child process (tests/variant_pkg.py)
 * the outputs of those merges are NaN (fp16 0x7E00) and nothing else;
 * va_merge_faults returns VA_ELOST with exactly one loss per merge group, and
   the next call returns VA_OK with 0 (each loss is reported once);
+* so for balanced paged batches, whose partials lie in ws, and those of equal lengths;
 * the ticket slot is left consistent: the same stream's next calls give up the
   same way (no stale count or tag carries over);
 * the two-pass form (S > 64: partials in ws, separate merge kernel) has no
@@ -97,6 +98,21 @@ def _child() -> None:
         assert np.all(got == 0x7E00), fmt.label
         assert faults() == (VA_ELOST, Hkv), fmt.label    # one per KV head (4 query heads: one sub-group)
         assert faults() == (VA_OK, 0)
+    # balanced paged batches, every merge group cut: counted with partials in ws (four and
+    # one query slots), and tagged for equal lengths with one slot
+    for fmt, Hq, lens in ((va.Fmt.Q8M, 8, [2100] * 4), (va.Fmt.F16M, 2, [9000, 9100, 8000, 7000]),
+                          (va.Fmt.F16M, 2, [9000] * 4)):
+        print(f"lost merge: balanced {fmt.label} Hq={Hq} {lens}", flush=True)
+        pb = batch_util.PagedBatch(fmt, lens, Hq, 2, 128, 32, 256, 0x10D2, max_seq_len=1 << 17, max_pages=512)
+        try:
+            for rep in range(2):
+                got = pb.run(stream=st)
+                assert (pb.ws_floats > 0) == (lens != [9000] * 4)
+                assert np.all(np.isnan(got)), (fmt.label, rep)
+                assert faults() == (VA_ELOST, 8), (fmt.label, rep)
+                assert faults() == (VA_OK, 0)
+        finally:
+            pb.free()
     # two-pass form: no in-kernel merge, nothing to lose
     fmt, H, L, S = va.Fmt.Q8M, 4, 3000, 80
     print(f"two-pass: {fmt.label} H={H} L={L} S={S}", flush=True)

@@ -76,13 +76,14 @@ def test_paged_d64_g64(fmt, page_rows):
 
 
 def test_paged_many_sequences_two_pass():
-    """B*Hq*S beyond the fused merge's partial store: the merge kernel path."""
-    lens = list(np.random.default_rng(3).integers(1, 600, 40))
+    """More merge groups than ticket lines: neither balanced nor fused, the merge kernel path."""
+    lens = list(np.random.default_rng(3).integers(1, 300, 130))
     pb = batch_util.PagedBatch(va.Fmt.Q8M, lens, 32, 8, 128, 32, 64, seed=11)
     try:
-        got = pb.run(S=4)           # 40*8 groups x 4 slots x 4 splits = 5120 partials > 2048
+        got = pb.run(S=4)           # 130 * 8 = 1040 merge groups > 1024
     finally:
         pb.free()
+    assert pb.ws_floats == 130 * 32 * 4 * (128 + 2)             # every split's partial
     for b in range(len(lens)):
         _check(got[b].ravel(), pb.ref[b].ravel(), b)
 

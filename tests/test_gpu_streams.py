@@ -152,7 +152,8 @@ def test_more_streams_than_ticket_slots(inputs):
 class Job:
     """One decode call with its own device inputs, enqueued on any stream into a
     caller-provided (out, ws) pair: one-slot (tagged merge), grouped (counted
-    merge, matrix-core and vector-ALU forms) or paged (counted merge)."""
+    merge, matrix-core and vector-ALU forms) or paged: static splits (counted merge), a
+    balanced batch (counted, partials in ws) or one of equal lengths (one slot: tagged)."""
 
     def __init__(self, kind, fmt, seed):
         from tests import batch_util
@@ -178,7 +179,10 @@ class Job:
             self.launch_args = (Hq, Hkv, L, D)
             self.out_heads = Hq
         else:
-            pb = batch_util.PagedBatch(fmt, [700, 1500, 64], 8, 2, D, G, 64, seed)
+            lens, Hq, cap = {"paged": ([700, 1500, 64], 8, None), "balanced": ([700, 5000, 64], 8, 1 << 17),
+                             "even": ([5000] * 4, 2, 1 << 17)}[kind]
+            pb = batch_util.PagedBatch(fmt, lens, Hq, 2, D, G, 64, seed, max_seq_len=cap,
+                                       max_pages=cap and cap // 64)
             self.pb = pb
             self.S = va.pick_splits_paged(fmt, pb.shape)
             quant = pb.kspool is not None
@@ -195,7 +199,7 @@ class Job:
         return va.ws_bytes(self.out_heads, self.D, self.S)
 
     def launch(self, out, ws, stream):
-        if self.kind == "paged":
+        if self.kind in ("paged", "balanced", "even"):
             b = va.PagedBufs(**self.bufs, out=out.ptr, ws=ws.ptr)
             va.decode_paged(self.fmt, b, self.pb.shape, self.S, stream=stream)
             return
@@ -210,17 +214,18 @@ class Job:
     def free(self):
         for x in self.dev:
             x.free()
-        if self.kind == "paged":
+        if self.kind in ("paged", "balanced", "even"):
             self.pb.free()
 
 
 def test_mixed_merge_protocols_on_concurrent_streams():
     """One-slot (tagged) and grouped / paged (counted) calls interleaved on four
-    streams while a captured graph of all four replays on a fifth: every output
+    streams while a captured graph of all replays on a fifth: every output
     equals its single-stream result bit for bit, and no merge is lost."""
     jobs = [Job("mha", va.Fmt.Q8M, 0x5A1), Job("gqa", va.Fmt.Q8M, 0x5A2),
-            Job("gqa", va.Fmt.F16M, 0x5A3), Job("paged", va.Fmt.Q4M, 0x5A4)]
-    assert all(j.S <= 64 for j in jobs)                       # all fused
+            Job("gqa", va.Fmt.F16M, 0x5A3), Job("paged", va.Fmt.Q4M, 0x5A4),
+            Job("balanced", va.Fmt.Q8M, 0x5A5), Job("even", va.Fmt.F16M, 0x5A6)]
+    assert all(j.S <= 64 for j in jobs[:4])                   # fused; the last two merge in the kernel with any S
     NS = 4
     streams = [va.Stream() for _ in range(NS)]
     gstream = va.Stream()

@@ -17,9 +17,12 @@ CUS = 256          # without a GPU, and on MI355X
 @pytest.mark.parametrize("L", [1, 4097, 10007, 262144])
 def test_groups_fit_whole_rounds(fmt, L):
     two = fmt in (va.Fmt.Q8M, va.Fmt.Q4M)
-    for H in range(1, 129):
+    for H in range(1, 256):
         S = va.pick_splits(fmt, H, L, 128)
         rounds = 2 if two and H * (CUS // H) < CUS - CUS // 32 and H * L >= 1280 * CUS else 1
+        if H > CUS // 2 and rounds == 1:        # rounded up: down would idle up to half the CUs
+            assert 1 <= S <= 2, (H, S)
+            continue
         assert 1 <= S and H * S <= rounds * CUS, (H, S)
         assert (S - 1) * va.split_chunk(L, S) < L, (H, S)            # no split is empty
     for Hkv in (1, 5, 6, 10, 12, 48, 100):
@@ -30,11 +33,17 @@ def test_groups_fit_whole_rounds(fmt, L):
 @pytest.mark.parametrize("B,Hq,Hkv", [(2, 32, 8), (16, 8, 8), (64, 32, 8), (100, 64, 8)])
 @pytest.mark.parametrize("L", [300, 16384, 1 << 20])
 def test_paged_splits_hold_pieces_and_pages(fmt, B, Hq, Hkv, L):
-    """The picked count keeps a split within the pages that a work-group stages (1024), for
-    calls that get no ticket slot, as well as giving the workspace of a balanced launch."""
+    """The picked count keeps a split, in whole kernel tiles (512 positions at most), within
+    the pages that a work-group stages (1024), for calls that get no ticket slot, as well as
+    giving the workspace of a balanced launch: a partial per merge group and per work-group."""
     shape = va.PagedShape(B, Hq, Hkv, 128, 32, 64, L // 64 + 1, 1 << 14, L)
     S = va.pick_splits_paged(fmt, shape)
-    assert S >= 1 and (-(-L // S) + 64) // 64 + 2 <= 1024, S
+    chunk = -(-(-(-L // 512)) // S) * 512
+    assert S >= 1 and chunk // 64 + 2 <= 1024, S
+    qg = min(4, Hq // Hkv)
+    groups = B * Hq // qg
+    if L < 1 << 20 and groups <= 1024 and (groups > CUS or groups * L >= 2048 * CUS):
+        assert B * Hq * S // qg >= groups + CUS, S
 
 
 @pytest.mark.gpu
