@@ -240,6 +240,11 @@ int groups_per_cu(int kind, bool tiled) {
 // against two (S 12) q8 20.7 -> 18.4 us, q4 14.7 -> 13.1; L 65536 107.5 -> 100.7 and 66.1
 // -> 57.7; H 20, L 20000 20.7 -> 19.8 and 14.7 -> 13.8. f16 is about even (H 40 33.9 ->
 // 32.5, H 24, L 8192 17.1 -> 18.2) and stays at one; two q3 groups do not fit a CU.
+// Where the line is not at its best: two gain with many heads (G 32, L 8192, H 100: q8
+// 40.1 -> 35.8, at D 64 21.9 -> 20.1; q4 23.6 -> 22.4, 14.6 -> 14.1) and cost with few or at
+// D 64 (H 12, L 65536: q8 34.8 -> 36.4, D 64 19.6 -> 20.6; q4 21.8 -> 24.2, 13.6 -> 15.0;
+// H 40, L 65536, D 64: q8 53.9 -> 54.2, q4 31.7 -> 33.3). Both are ahead of rounding the
+// splits up to a partial second round (H 12: q4 29.3, D 64 17.0; H 40, D 64 41.9).
 bool two_groups_fit(int kind) { return kind == KQ8 || kind == KQ4; }
 
 template <int KIND, int D, int G>

@@ -124,12 +124,14 @@ static int max_tile() {
 // more merge groups than CUs, when a run begins several of them and one group's start
 // and end hide behind the other's loop (batch of 64 up to 3000 positions, Hq 32 / Hkv 8:
 // q4 36.0 -> 30.5 us, q3 39.2 -> 34.2; eight waves stay better for q8, uniform batch of 32
-// x 4096 56.3 -> 50.3, and with fewer merge groups; with exactly one per CU eight lose on
-// uneven lengths what four lose on equal ones: 32 up to 16384 q4 43.3 -> 49.1, 32 x 4096
-// 38.3 -> 32.2, and eight are nowhere behind what was there before four were). Vector ALU with one query slot
-// (4-wave groups): two per CU (batch of 64 up to 2000, Hkv 8: q8 25.1 -> 20.3 us, q3 24.9 ->
-// 20.8, f16 32.9 -> 31.1; batch of 16 up to 8192 q8 17.4 -> 15.4), one where fewer merge
-// groups meet longer items (q4 at D 128 16.5 against 18.0, D 64 q8 13.5 against 15.1).
+// x 4096 56.3 -> 50.3, and with fewer merge groups). With exactly one merge group per CU
+// four gain on uneven lengths what they lose on equal ones, and eight are behind neither
+// form of before: q4 32 up to 16384 43.3 (4 waves) against 49.1 (static splits 110), 32 x
+// 4096 38.3 against 32.2 (36.0).
+// Vector ALU with one query slot (4-wave groups): two per CU (batch of 64 up to 2000, Hkv
+// 8: q8 25.1 -> 20.3 us, q3 24.9 -> 20.8, f16 32.9 -> 31.1; batch of 16 up to 8192 q8 17.4 ->
+// 15.4), one where fewer merge groups meet longer items (q4 at D 128 16.5 against 18.0, D
+// 64 q8 13.5 against 15.1; f16 and q3 at D 64 were not measured apart).
 // Grouped f16 and q3 at D = 64 (8-wave groups): one (f16 26.1 against 34.1).
 int balanced_waves(int kind, long long groups, int cus) { return kind != KQ8 && groups > cus ? 4 : 8; }
 

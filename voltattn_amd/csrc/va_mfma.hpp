@@ -42,10 +42,10 @@
 // Softmax: log2 units (q pre-scaled by log2(e)/sqrt(D) in fp32 after the dot),
 // lazy running maximum per query slot as in decode_tiled (RESCALE_SLACK).
 //
-// Work split, loads and the merge are decode_tiled's: one work-group per
-// (merge group, split), or per run of a balanced paged batch (BAL, va_balance.hpp), per-wave 32-row tiles double-buffered in registers,
-// buffer resources bounded by the split (or per tile for paged caches), and
-// finish_partial for the partials / fused merge.
+// Work split, loads and the merge are decode_tiled's: one work-group per (merge group,
+// split), or per run of a balanced paged batch (BAL, va_balance.hpp), per-wave 32-row tiles
+// double-buffered in registers, buffer resources bounded by the split (or per tile for
+// paged caches), and finish_partial for the partials / fused merge.
 #pragma once
 #include "va_codec.hpp"
 #include "va_balance.hpp"

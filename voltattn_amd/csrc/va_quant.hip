@@ -43,10 +43,10 @@ template <class T>
 __device__ __forceinline__ void stream_store(T* p, T v) { __builtin_nontemporal_store(v, p); }
 
 // Codes of E values against the group scale sh (its fp16 value): bit-exact with
-// clamp(rint(x / sh)), a non-finite quotient giving 0. x * rcp(sh) is within 2^-22
-// of the IEEE quotient, relatively, so within 2^-15 absolutely (|quotient| < 192: a scale that rounds
-// down to an fp16 subnormal may be two thirds of amax / lim):
-// where no value lies that close to a rounding boundary (and none is NaN or
+// clamp(rint(x / sh)), a non-finite quotient giving 0. x * rcp(sh) is within 2^-22 of the
+// IEEE quotient, relatively. A quotient of lim + 1 or more clamps whichever side of a
+// boundary it lands; below, |quotient| < 128, so the two differ by less than 2^-15:
+// where no value lies within 2^-14 of a rounding boundary (twice that; and none is NaN or
 // infinite), rounding it gives the same code; otherwise the wave divides.
 template <int BITS, int E>
 __device__ __forceinline__ void quant_codes(const float (&x)[E], float sh, int (&code)[E]) {

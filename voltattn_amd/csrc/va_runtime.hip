@@ -273,7 +273,9 @@ int cus_or_default() {
 // many as fit in one round. (One more each, which the reference's rule rounds up to,
 // leaves a few work-groups for a second round: H 40, D 128, G 64 on MI355X, S 7 -> 6,
 // L 10007: q3 20.7 -> 13.0 us, f16 41.3 -> 33.9.) Above half the slots rounding down
-// would idle up to half of them, and the groups are many enough to overlap.
+// would idle up to half of them, so it rounds up: H 132, D 128, G 32, S 1 -> 2: q8 L 8192
+// 69.5 -> 53.3, L 65536 530.7 -> 402.2; f16 about even (105.5 -> 105.5, 821.0 -> 834.9);
+// q3 alone loses (34.9 -> 40.7, 240.4 -> 252.1).
 int whole_splits(int slots, int groups) {
     return std::max(1, 2 * groups <= slots ? slots / groups : (slots + groups - 1) / groups);
 }
@@ -502,14 +504,15 @@ void splits_ex(int kind, int D, int qg, int groups, int max_len, int S_req, int*
 // Work-groups of the balanced form (va_balance.hpp) for a paged batch, or 0 where
 // every merge group is cut into S splits of the longest sequence instead.
 //
-// The plan costs a launch 1 to 2 us, so it is for batches whose uneven lengths can cost
+// The plan costs a launch about 1 us, so it is for batches whose uneven lengths can cost
 // more than that: more merge groups than CUs (a split each leaves a half-empty last
-// round), or at least 2048 positions per CU. Measured on MI355X against the splits, D
-// 128, lengths spread over 1/32 .. 1 of the longest: q8 batch of 48 up to 16384, Hq 32 /
-// Hkv 8 171 -> 104 us; q4 64 up to 3000 43.7 -> 30.6; f16 16 up to 8000 63.8 -> 26.1; Hq =
-// Hkv = 8, 16 up to 8192 f16 56.6 -> 22.6, q8 39.6 -> 15.4; Hq 64 / Hkv 8 q4 63.1 -> 26.7.
-// Equal lengths: 40 x 2048 q8 53.8 -> 41, 32 x 4096 52.0 -> 51.2, 8 x 16384 51.8 -> 53.2;
-// below the line 4 x 8192 with Hq = Hkv = 8 would be 15.0 -> 17.2, 2 x 512 6.7 -> 9.0.
+// round), or at least 2048 positions per CU. Measured on MI355X, static splits ->
+// balanced, D 128, lengths spread over 1/32 .. 1 of the longest: Hq 32 / Hkv 8, 16 up to
+// 8192 q8 42.5 -> 25.2 us, q4 36.1 -> 22.2, q3 43.0 -> 23.8, f16 64.7 -> 32.6; 64 up to 3000
+// q8 51.0 -> 37.5, q4 44.9 -> 26.6; 32 up to 16384 q8 139 -> 59, f16 232 -> 95; Hq = Hkv = 8,
+// 16 up to 8192 f16 58.2 -> 30.2, q8 40.1 -> 19.8. Equal lengths: DecodeArgs::even
+// (va_balance.hpp), or 40 x 2048, Hq 32 / Hkv 8 q8 53.2 -> 40.5; below the line 4 x 8192
+// with Hq = Hkv = 8 would be 15.0 -> 17.2, 2 x 512 6.7 -> 9.0.
 //
 // Also 0: one sequence (its length is what the splits are made for), more merge groups
 // than ticket lines, a run that could span more pages than a work-group stages, or a
