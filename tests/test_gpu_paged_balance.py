@@ -64,7 +64,8 @@ def test_more_merge_groups_than_cus(fmt, heads):
     B = 70 if Hkv == 8 else 140
     lens = _ragged(3, B, 400)
     lens[5] = lens[6] = lens[B - 1] = 0
-    assert _run(fmt, lens, Hq, Hkv, 128, 32, 64, seed=Hq) > 0
+    cap = 2048 if Hq == Hkv else None            # one query slot: short capacities keep static splits
+    assert _run(fmt, lens, Hq, Hkv, 128, 32, 64, seed=Hq, max_seq_len=cap) > 0
 
 
 @pytest.mark.parametrize("fmt", TILED, ids=lambda f: f.label)
@@ -131,7 +132,7 @@ def test_invalid_lengths_and_pages(case, cut):
         lens, cap = [3000, 400, 0, 900, 2500, 5000, 9000, 7000], 1 << 17
     else:
         lens = [90, 300, 0, 280, 300, 200, 310, 250] + _ragged(6, 36 if Hkv == 8 else 140, 320)
-        cap = 320
+        cap = 2048 if Hq == Hkv else 320
     for page in (-1, 1 << 20):
         pb = batch_util.PagedBatch(fmt, lens, Hq, Hkv, 128, 32, P, seed=Hq + P, max_seq_len=cap, max_pages=-(-cap // P))
         try:
@@ -144,6 +145,16 @@ def test_invalid_lengths_and_pages(case, cut):
         for b in (1, 3, 5, 6, 7):
             assert np.all(np.isnan(got[b])), b
         _check_batch(pb, got, skip=(1, 3, 5, 6, 7))
+
+
+@pytest.mark.parametrize("fmt,D,cap", [(va.Fmt.F16M, 128, 1024), (va.Fmt.Q8M, 128, 1024), (va.Fmt.Q4M, 128, 1536),
+                                       (va.Fmt.Q3M, 128, 1536), (va.Fmt.Q8M, 64, 2048)],
+                         ids=lambda x: x.label if isinstance(x, va.Fmt) else str(x))
+@pytest.mark.parametrize("less", [0, 1])
+def test_one_slot_short_capacities_keep_static_splits(fmt, D, cap, less):
+    """One work-group per merge group below the line, whose partial stays in the kernel."""
+    wrote = _run(fmt, _ragged(5, 40, 300), 8, 8, D, 32, 64, seed=cap + D, max_seq_len=cap - less)
+    assert wrote == 0 if less else wrote > 0, wrote
 
 
 def test_without_a_ticket_slot():
@@ -173,7 +184,7 @@ def test_small_workspaces(S):
 def test_captured_step_follows_the_lengths(fmt, Hq):
     Hkv, D, G, P = 8, 128, 32, 64
     full = _ragged(4, 36, 700)
-    pb = batch_util.PagedBatch(fmt, full, Hq, Hkv, D, G, P, seed=77)
+    pb = batch_util.PagedBatch(fmt, full, Hq, Hkv, D, G, P, seed=77, max_seq_len=2048, max_pages=2048 // P)
     st = va.Stream()
     try:
         B = len(full)

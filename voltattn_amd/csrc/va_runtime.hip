@@ -514,12 +514,21 @@ void splits_ex(int kind, int D, int qg, int groups, int max_len, int S_req, int*
 // (va_balance.hpp), or 40 x 2048, Hq 32 / Hkv 8 q8 53.2 -> 40.5; below the line 4 x 8192
 // with Hq = Hkv = 8 would be 15.0 -> 17.2, 2 x 512 6.7 -> 9.0.
 //
+// With one query slot a work-group per merge group is as short as its sequence, and the
+// hardware's dispatch of many short ones evens them out by itself: up to 1024 positions of
+// q8 and f16, and 1536 of q4 and q3, at D 128 (twice that at D 64) static splits stay.
+// Hq = Hkv = 8, static -> balanced: 64 up to 300 q4 9.8 -> 15.0, q3 9.6 -> 15.4, q8 9.3 -> 13.1,
+// f16 9.8 -> 13.5; 64 up to 1024 q4 15.2 -> 18.0, q3 15.7 -> 17.1, q8 17.1 -> 16.1, f16 23.0 ->
+// 19.6; 128 up to 2000 q4 31.0 -> 29.1, q3 31.5 -> 30.3; D 64, 128 up to 1024 q8 14.5 -> 18.6.
+// (A capacity far above the lengths hides this from the rule.)
+//
 // Also 0: one sequence (its length is what the splits are made for), more merge groups
 // than ticket lines, a run that could span more pages than a work-group stages, or a
 // workspace of S splits (S = 0: any) too small for the pieces of one run per CU.
 int balanced_wgs(int kind, const va_paged_shape* sh, int qg, long long groups, int S, int cus) {
     if (sh->B < 2 || groups > va::TICKET_MAXH) return 0;
     if (groups <= cus && groups * sh->max_seq_len < 2048LL * cus) return 0;
+    if (qg == 1 && (long long)sh->max_seq_len * sh->D < (kind == 2 || kind == 3 ? 1536 : 1024) * 128LL) return 0;
     long long n = va::balanced_groups(kind, sh->D, qg, groups, cus);
     n = std::min(n, (long long)va::MAX_RUNS);
     if (S > 0) n = std::min(n, (long long)sh->B * sh->Hq * S / qg - groups);
